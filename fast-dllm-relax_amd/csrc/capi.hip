@@ -324,6 +324,11 @@ int plan_attention(fdllm_ctx* c, AttnP& a, int rows, uint16_t* kc, uint16_t* vc,
   a.mask = mask; a.q_pos0 = 0; a.block = f.bd_size; a.bias = bias; a.bias_ld = bias_ld;
   a.nseq = 1;
   int target = c->attn_target;
+  if (sb != nullptr && sb->nseq == 1) {
+    // a batch of one sequence is that sequence's own call: it takes the one-sequence kernels below
+    a.rows = sb->rows; a.ws = sb->ws[0]; a.Lk = sb->lk[0];
+    sb = nullptr;
+  }
   if (sb != nullptr) {
     a.nseq = sb->nseq; a.rows = sb->rows; a.seq_stride = sb->seq_stride;
     a.ws = 0; a.Lk = 0;

@@ -288,3 +288,23 @@ def test_batched_step_ragged_query_tiles(wide2):
         bf16_parity(f"{R}-row batched vs batch-1, sequence {b} hidden", to_np(h[b]), to_np(hb[0]))
         bf16_parity(f"{R}-row batched vs batch-1, sequence {b} K rows", to_np(k[:, b, P:P + R]),
                     to_np(kb[:, 0, P:P + R]))
+
+
+@pytest.mark.parametrize("rows,prefix", [(32, 32), (32, 500), (32, 6000), (64, 300), (130, 70)])
+def test_batch_of_one_is_the_sequences_own_call(tiny, rows, prefix):
+    """A batch of one sequence plans its attention as that sequence's forward_cached does (its key splits'
+    partials sized for them): the same bits in the hidden states and in the caches."""
+    _, vm = tiny
+    L, nkv, hd = TINY["num_hidden_layers"], TINY["num_key_value_heads"], TINY["head_dim"]
+    cap = prefix + rows + 32
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows + prefix)
+    k = torch.randn((L, 1, cap, nkv, hd), device="cuda", generator=g).to(vm.torch_dtype)
+    v = torch.randn((L, 1, cap, nkv, hd), device="cuda", generator=g).to(vm.torch_dtype)
+    x = vm.embed(torch.randint(0, 999, (rows,), dtype=torch.int32, device="cuda", generator=g))[None]
+    k1, v1, k2, v2 = k.clone(), v.clone(), k.clone(), v.clone()
+    log(f"case: one sequence of {rows} rows at {prefix}, as a batch of one and alone")
+    h1 = vm.forward_cached_batch(x, k1, v1, torch.tensor([prefix], dtype=torch.int32, device="cuda"), [prefix])
+    h2 = vm.forward_cached(x, k2, v2, torch.tensor(prefix, dtype=torch.int32, device="cuda"), prefix)
+    for name, a, b in (("hidden", h1, h2), ("k", k1, k2), ("v", v1, v2)):
+        np.testing.assert_array_equal(to_np(a), to_np(b), err_msg=name)
