@@ -14,15 +14,65 @@ namespace fdllm {
 // then runs over other blocks, which changes the rounding; batched calls on 2 tiles: 128-row partial
 // step 2.73 against 2.54 ms.)
 
+// the prefill kernel takes row blocks of at least this many rows without an explicit bias
+constexpr int PREFILL_MIN_ROWS = 128;
+
+// one sequence's unmasked call takes attn_seq_kernel below this many rows (us per layer over 8175 keys, the
+// loop kernel up to 127 rows and the one-block prefill kernel from there / this one: 48 rows 69 / 19, 83
+// rows 168 / 23, 127 rows 221 / 30, 300 rows 185 / 60, 600 rows 193 / 100; over 256 keys 12.5 / 9.9, 16.4 /
+// 10.9, 19.6 / 11.3, 20.2 / 17.6, 27.4 / 17.7)
+constexpr int SEQ_ONE_MAX_ROWS = 1024;
+
+// attn_seq_kernel: key blocks ahead, waves (key parts) per query tile and query tiles per workgroup.
+constexpr int SEQ_DEPTH = 3;
+#ifndef FD_SEQ_KH
+#define FD_SEQ_KH 2
+#endif
+#ifndef FD_SEQ_NQW
+#define FD_SEQ_NQW 2
+#endif
+constexpr int SEQ_KH = FD_SEQ_KH, SEQ_NQW = FD_SEQ_NQW;
+
+// One sequence on attn_seq_kernel: S key splits (merged by attn_merge_kernel), and its qg query-tile
+// groups dealt to the XCDs in xh runs.  A unit is one run of one (split, kv head): its workgroups share
+// the split's K/V through one XCD's L2, so whole units go to an XCD and an XCD with more units than the
+// others sets the time (64 rows over 8100 keys: 10 splits in one run each 31.6 us, 8 splits 21.1).  The
+// choice is the cheapest of, per xh, no split and as many splits as one workgroup per compute unit
+// allows, at the measured 1 us per 64-key block, 3 us per round of workgroups, 4.5 us for the merge launch
+// and 4.2 ns per partial tile written and read back.
+constexpr int SEQ_ONE_MAX_SPLITS = 40, SEQ_ONE_MAX_RUNS = 8;
+static void seq_one_splits(AttnPlan& p, int QT, int nkv, int Lk, int ncu) {
+  const int T = (Lk + 63) / 64, per_xcd = std::max(1, ncu / 8);
+  float best = 0.f;
+  p.S = p.xh = 0;
+  for (int xh = 1; xh <= SEQ_ONE_MAX_RUNS; ++xh) {
+    const int wgs = (p.qg + xh - 1) / xh;  // of one unit
+    for (const int S : {1, std::min({per_xcd / wgs * 8 / (nkv * xh), T / 2, SEQ_ONE_MAX_SPLITS})}) {
+      if (S < 1) continue;
+      const int rounds = ((S * nkv * xh + 7) / 8 * wgs + per_xcd - 1) / per_xcd;
+      const float cost = (float)(rounds * ((T + S - 1) / S + 3)) + (S > 1 ? 4.5f + 0.0042f * (float)(S * QT * nkv) : 0.f);
+      if (p.S == 0 || cost < best) {
+        best = cost;
+        p.S = S;
+        p.xh = xh;
+      }
+    }
+  }
+}
+
 // Launch plan: short row blocks (the cached decode step) use attn_chunk_kernel with one key chunk of
 // CH keys per workgroup; long row blocks (prefill, stateless forward) use attn_kernel with few, long
 // key ranges per workgroup.
-AttnPlan attn_plan(int rows, int nq, int nkv, int Lk, int target_wgs, int nseq) {
+AttnPlan attn_plan(int rows, int nq, int nkv, int Lk, int target_wgs, int nseq, int mask, int ncu) {
   AttnPlan p{};
   const int QT = ((nq / nkv) * rows + 15) / 16;
+  const bool seq = nseq <= 1 && mask == 0 && ncu > 0 && rows < SEQ_ONE_MAX_ROWS;
   // chunked: 128 keys per workgroup unless that leaves fewer workgroups than aimed for; at most 64
-  // chunks, so the split merge stays small (longer contexts take the loop kernel)
-  if (QT <= 12 && (Lk + 127) / 128 <= 64) {
+  // chunks, so the split merge stays small (longer contexts take the loop kernel), and at most 40 where
+  // attn_seq_kernel can take the call: past the splits its merge reads in one round trip the chunk kernel
+  // falls behind (rotated queries, 32 rows: 18.1 / 18.5 us at 4096 keys, 29.0 / 20.0 at 6000, 33.0 / 22.8
+  // at 8100; 8 rows: 13.6 / 12.9, 19.3 / 13.4, 22.8 / 14.3; the RoPE and append pass of a step adds 4.5 us)
+  if (QT <= 12 && (Lk + 127) / 128 <= (seq ? 40 : 64)) {
     p.chunked = 1;
     p.key_groups = 2;
     p.chunk = 128;
@@ -33,6 +83,15 @@ AttnPlan attn_plan(int rows, int nq, int nkv, int Lk, int target_wgs, int nseq) 
     return p;
   }
   p.chunked = 0;
+  if (seq) {
+    p.seq = 1;
+    p.q_tiles_per_wg = SEQ_NQW;
+    p.key_groups = SEQ_KH;
+    p.qg = (QT + SEQ_NQW - 1) / SEQ_NQW;
+    p.chunk = 64;
+    seq_one_splits(p, QT, nkv, Lk, ncu);
+    return p;
+  }
   if (QT >= 32) { p.q_tiles_per_wg = 4; p.key_groups = 1; }
   else { p.q_tiles_per_wg = 4; p.key_groups = 2; }
   p.qg = (QT + p.q_tiles_per_wg - 1) / p.q_tiles_per_wg;
@@ -176,20 +235,7 @@ static hipError_t launch_prefill(const AttnP& a, hipStream_t st) {
   }
 }
 
-// the prefill kernel takes row blocks of at least this many rows without an explicit bias
-constexpr int PREFILL_MIN_ROWS = 128;
-
-// Batched calls without a mask: the RoPE + KV append pass over the call's rows, then attn_seq_kernel with
-// its key blocks SEQ_DEPTH ahead and SEQ_KH key parts (waves per query tile).
-constexpr int SEQ_DEPTH = 3;
-#ifndef FD_SEQ_KH
-#define FD_SEQ_KH 2
-#endif
-#ifndef FD_SEQ_NQW
-#define FD_SEQ_NQW 2
-#endif
-constexpr int SEQ_KH = FD_SEQ_KH, SEQ_NQW = FD_SEQ_NQW;
-
+// Batched calls without a mask: the RoPE + KV append pass over the call's rows, then attn_seq_kernel.
 size_t plan_seq_units(AttnP& a, int ncu) {
   const int QT = ((a.nq / a.nkv) * a.rows + 15) / 16, xg = (QT + SEQ_NQW - 1) / SEQ_NQW;
   int T[MAX_SEQS], s[MAX_SEQS];
@@ -232,27 +278,36 @@ size_t plan_seq_units(AttnP& a, int ncu) {
 
 template <int DT>
 static hipError_t launch_seq(const AttnP& a, hipStream_t st) {
-  if (a.nunits < a.nseq || a.nunits > MAX_SEQ_UNITS) return hipErrorInvalidValue;
-  if (!a.roped) hipLaunchKernelGGL(rope_kv_kernel<DT>, dim3(a.nseq * a.rows), dim3(128), 0, st, a);
+  const bool one = a.nseq <= 1;
+  if (one ? a.S < 1 || a.S > (a.Lk + 63) / 64 : a.nunits < a.nseq || a.nunits > MAX_SEQ_UNITS) return hipErrorInvalidValue;
+  if (!a.roped) hipLaunchKernelGGL(rope_kv_kernel<DT>, dim3((one ? 1 : a.nseq) * a.rows), dim3(128), 0, st, a);
   const int QT = ((a.nq / a.nkv) * a.rows + 15) / 16, xg = (QT + SEQ_NQW - 1) / SEQ_NQW;
-  const int pairs = a.nunits * a.nkv;
+  const int xh = one ? a.xh : 1, xs = (xg + xh - 1) / xh;
+  if (xh < 1) return hipErrorInvalidValue;
+  const int units = (one ? a.S : a.nunits) * a.nkv * xh;
   auto kern = attn_seq_kernel<DT, SEQ_DEPTH, SEQ_NQW, SEQ_KH>;
   constexpr size_t lds = (size_t)(SEQ_DEPTH + 1) * 2 * 64 * HD * 2;  // K and V of D + 1 key blocks
   raise_lds(kern, lds);
-  hipLaunchKernelGGL(kern, dim3((pairs + 7) / 8 * 8 * xg), dim3(64 * SEQ_NQW * SEQ_KH), lds, st, a);
+  hipLaunchKernelGGL(kern, dim3((units + 7) / 8 * 8 * xs), dim3(64 * SEQ_NQW * SEQ_KH), lds, st, a);
+  if (one && a.S > 1) hipLaunchKernelGGL(merge_kernel_for<DT>(a.S), dim3(HD / 16, QT, a.nkv), dim3(64), 0, st, a);
   return hipGetLastError();
 }
 
 bool attn_takes_roped(const AttnP& a) {
   if (a.nseq > 1 && a.seq_attn && a.mask == 0) return true;
-  const AttnPlan p = attn_plan(a.rows, a.nq, a.nkv, a.Lk, a.target_wgs, a.nseq);
+  if (a.nseq <= 1 && a.seq_attn) return true;
+  const AttnPlan p = attn_plan(a.rows, a.nq, a.nkv, a.Lk, a.target_wgs, a.nseq, a.mask, a.ncu);
   return !p.chunked && a.nseq <= 1 && a.rows >= PREFILL_MIN_ROWS && a.mask != 2;
 }
 
 template <int DT>
 static hipError_t launch_dt(const AttnP& a, hipStream_t st) {
-  const AttnPlan p = attn_plan(a.rows, a.nq, a.nkv, a.Lk, a.target_wgs, a.nseq);
-  if (a.roped && !attn_takes_roped(a)) return hipErrorInvalidValue;
+  if (a.nseq <= 1 && a.seq_attn) {
+    if (a.mask != 0 || (a.ofrag && a.rows > 32)) return hipErrorInvalidValue;
+    return launch_seq<DT>(a, st);
+  }
+  const AttnPlan p = attn_plan(a.rows, a.nq, a.nkv, a.Lk, a.target_wgs, a.nseq, a.mask, a.ncu);
+  if (p.seq || (a.roped && !attn_takes_roped(a))) return hipErrorInvalidValue;
   if (p.S != a.S || p.chunk != a.chunk) return hipErrorInvalidValue;
   if (a.ofrag && (a.nseq > 1 || a.rows > 32)) return hipErrorInvalidValue;
   if (a.nseq > MAX_SEQS) return hipErrorInvalidValue;

@@ -809,7 +809,7 @@ __device__ __forceinline__ void rope_kv_row(const AttnP& a, int r) {
       u32x4 lo = *reinterpret_cast<const u32x4*>(hs + 8 * p);
       u32x4 hi = *reinterpret_cast<const u32x4*>(hs + 64 + 8 * p);
       rope_tab<DT>(lo, hi, cs + 16 * p);
-      u16* dst = hd < a.nq ? a.out + (size_t)r * a.nq * HD + hd * HD
+      u16* dst = hd < a.nq ? (a.qrot != nullptr ? a.qrot + (size_t)r * a.ldqr : a.out + (size_t)r * a.nq * HD) + hd * HD
                            : a.kc + (size_t)(a.ws + r) * krow + (hd - a.nq) * HD;
       *reinterpret_cast<u32x4*>(dst + 8 * p) = lo;
       *reinterpret_cast<u32x4*>(dst + 64 + 8 * p) = hi;
@@ -1329,9 +1329,15 @@ void attn_prefill_pair_kernel(AttnP a) {
 // block: the scores of block t + 1 are formed while block t's softmax and P.V run (same arithmetic and
 // order per block; measured 16.8 -> 16.0 us per layer on the 512-row batched step).
 // A sequence of one split writes its output directly; splits merge as described at the end.
+// One sequence's unmasked call (nseq <= 1: scoring, a block after more keys than the chunk kernel takes)
+// runs here too, split into p.S equal ranges of key blocks whose partials attn_merge_kernel combines: the
+// loop kernel it replaces aimed for 64 workgroups and waited out a memory round trip per 32 keys (83 rows
+// over 8275 keys: 168 -> 23 us; 32 rows: 47 -> 23).  What bounds it is the serial chain of a block in one
+// wave per SIMD (scores, softmax, P.V: about 1 us per 64 keys), not the 8.5 MB of K and V.
 // 1-D grid in XCD-aware order: linear index i, slot i % 8, round i / 8; pair (u, g) = (round / XG) x 8 +
 // slot, query group x = round % XG, so the XG workgroups that read one split's K/V run on one XCD and
-// share its L2.  Indices past the last pair have nothing to do.
+// share its L2.  Indices past the last pair have nothing to do.  (One sequence: runs of XG / p.xh groups
+// instead of whole pairs, seq_one_splits.)
 template <int DT, int D, int NQW, int KH>
 __global__ __launch_bounds__(64 * NQW * KH) __attribute__((amdgpu_waves_per_eu(NQW * KH > 4 ? 2 : 1, NQW * KH > 4 ? 2 : 1)))
 void attn_seq_kernel(AttnP p) {
@@ -1349,20 +1355,31 @@ void attn_seq_kernel(AttnP p) {
   extern __shared__ __align__(16) unsigned char smem[];
 
   const int grp = p.nq / p.nkv, QR = grp * p.rows, QT = (QR + 15) / 16, XG = (QT + NQW - 1) / NQW;
+  const bool one = p.nseq <= 1;
+  const int XH = one ? p.xh : 1, XS = (XG + XH - 1) / XH;
   const int i = blockIdx.x, round = i >> 3;
-  const int pair = (round / XG) * 8 + (i & 7), x = round % XG;
-  if (pair >= p.nunits * p.nkv) return;
+  const int unit = (round / XS) * 8 + (i & 7), pair = unit / XH, x = (unit - pair * XH) * XS + round % XS;
+  if (pair >= (one ? p.S : p.nunits) * p.nkv || x >= XG) return;
   const int u = pair / p.nkv, g = pair - u * p.nkv;
-  const int ua = p.unit_a[u], ut = p.unit_t[u];
-  const int b = ua & 63, js = (ua >> 6) & 31, ns = (ua >> 11) & 31, u0 = ua >> 16;  // partials at u0 + js
-  const int tb = ut & 0xffff;  // this split's key blocks [tb, tb + T)
   AttnP a = p;
-  seq_view(a, p, b);
+  int b = 0, js = u, ns = p.S, u0 = 0;  // split js of ns; partials at u0 + js
+  int tb, te;                           // this split's key blocks [tb, te)
+  if (one) {
+    const int nb = (p.Lk + KBP - 1) / KBP;
+    tb = nb * js / ns;
+    te = nb * (js + 1) / ns;
+  } else {
+    const int ua = p.unit_a[u], ut = p.unit_t[u];
+    b = ua & 63; js = (ua >> 6) & 31; ns = (ua >> 11) & 31; u0 = ua >> 16;
+    tb = ut & 0xffff;
+    te = ut >> 16;
+    seq_view(a, p, b);
+  }
 
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int qw = w % NQW, kh = w / NQW;
   const int lr = lane & 15, lg = lane >> 4;
-  const int Lk = a.Lk, T = (ut >> 16) - tb;
+  const int Lk = a.Lk, T = te - tb;
   const size_t krow = (size_t)a.nkv * HD;
   const u16* kc = a.kc + g * HD + (size_t)tb * KBP * krow;  // block t of the split: the sequence's tb + t
   const u16* vc = a.vc + g * HD + (size_t)tb * KBP * krow;
@@ -1410,7 +1427,7 @@ void attn_seq_kernel(AttnP p) {
   const int r = qvalid ? qi - hh * a.rows : 0;
   u32x4 qf[4];
   {
-    const u16* qp = a.out + (size_t)r * a.nq * HD + (g * grp + hh) * HD + 8 * lg;
+    const u16* qp = (a.qrot != nullptr ? a.qrot + (size_t)r * a.ldqr : a.out + (size_t)r * a.nq * HD) + (g * grp + hh) * HD + 8 * lg;
 #pragma unroll
     for (int ds = 0; ds < 4; ++ds) qf[ds] = *reinterpret_cast<const u32x4*>(qp + 32 * ds);
   }
@@ -1573,6 +1590,7 @@ void attn_seq_kernel(AttnP p) {
 
   float L = l_run;
   float Mw = m_run == -INFINITY ? 0.f : m_run;  // o and L are relative to 2^Mw
+  float Mr = m_run;                             // the maximum itself
   if constexpr (KH > 1) {
     // merge the key parts in LDS, in part order (the chunk kernel's merge): parts > 0 leave (m, l) and O^T,
     // part 0 combines them
@@ -1594,6 +1612,7 @@ void attn_seq_kernel(AttnP p) {
     for (int k = 0; k < KH; ++k) M = fmaxf(M, cm[(k * NQW + qw) * 16 + lr]);
     const float Mu = M == -INFINITY ? 0.f : M;
     Mw = Mu;
+    Mr = M;
     L = 0.f;
     for (int k = 0; k < KH; ++k) L += cl[(k * NQW + qw) * 16 + lr] * __builtin_amdgcn_exp2f(cm[(k * NQW + qw) * 16 + lr] - Mu);
     const float f0 = __builtin_amdgcn_exp2f(cm[qw * 16 + lr] - Mu);
@@ -1604,6 +1623,16 @@ void attn_seq_kernel(AttnP p) {
 #pragma unroll
       for (int dt = 0; dt < DT16; ++dt) o[dt] += co[(((k - 1) * NQW + qw) * DT16 + dt) * 64 + lane] * fk;
     }
+  }
+  if (one && ns > 1) {
+    // one sequence's key splits: partials in the layout attn_merge_kernel, launched next, combines (a last
+    // arriver would read up to 40 splits of 8 KB alone; the merge spreads them over 8 waves per tile)
+    if (tile >= QT) return;
+    float* pp = p.part + ((size_t)(g * QT + tile) * ns + js) * PSZ;
+#pragma unroll
+    for (int dt = 0; dt < DT16; ++dt) reinterpret_cast<f32x4*>(pp)[dt * 64 + lane] = o[dt];
+    if (lg == 0) *reinterpret_cast<f32x2_t*>(pp + 16 * HD + 2 * lr) = f32x2_t{Mr, L};
+    return;
   }
   if (ns > 1) {
     // key splits: every split's wave leaves (O, m, l) of its query tile by write-through stores; the last to
@@ -1646,10 +1675,9 @@ void attn_seq_kernel(AttnP p) {
   }
   if (!qvalid) return;
   const float inv = 1.0f / L;
-  u16* dst = a.out + (size_t)r * a.nq * HD + (g * grp + hh) * HD + 4 * lg;
 #pragma unroll
   for (int dt = 0; dt < DT16; ++dt)
-    *reinterpret_cast<u32x2*>(dst + 16 * dt) =
+    *reinterpret_cast<u32x2*>(out_at(a, r, (g * grp + hh) * HD + 4 * lg + 16 * dt)) =
         u32x2{pack_f32x2<DT>(o[dt][0] * inv, o[dt][1] * inv), pack_f32x2<DT>(o[dt][2] * inv, o[dt][3] * inv)};
 }
 

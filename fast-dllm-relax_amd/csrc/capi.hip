@@ -100,7 +100,8 @@ struct fdllm_ctx {
   int attn_target = 64;   // attention workgroups aimed for when splitting the keys
   int prefill_hpw = 0;    // query heads per prefill-attention workgroup (0: chosen per launch)
   int prefill_pair = 1;   // paired-query-block prefill attention (0 off, 1 by size, 2 always all heads, 3 always split)
-  int seq_attn = 1;       // batched calls: attn_seq_kernel (0: the chunk kernel with key splits + merge)
+  int seq_attn = 1;       // attn_seq_kernel for batched calls and one sequence's longer ones (0: the chunk kernel with
+                          // key splits + merge, the loop kernel and the prefill kernel)
   int seq_split = 1;      // attn_seq_kernel splits long sequences' keys over the compute units it leaves idle
   int ncu = 256;          // compute units of the device
   unsigned* attn_cnt = nullptr;  // attn_seq_kernel's arrival counters (SEQ_CNT_MAX, zero between launches)
@@ -338,7 +339,8 @@ int plan_attention(fdllm_ctx* c, AttnP& a, int rows, uint16_t* kc, uint16_t* vc,
     }
     target = std::max(1, target / sb->nseq);
   }
-  const AttnPlan pl = attn_plan(a.rows, a.nq, a.nkv, a.Lk, target, a.nseq);
+  a.ncu = c->seq_attn ? c->ncu : 0;
+  const AttnPlan pl = attn_plan(a.rows, a.nq, a.nkv, a.Lk, target, a.nseq, mask, a.ncu);
   // batched calls without a mask take attn_seq_kernel (every key of a sequence in one workgroup, no
   // partials) from 32 rows per sequence, or when the chunk plan cannot cover the longest sequence in one
   // step; otherwise the chunk kernel.  Measured on config 4 (16 sequences, prefixes up to 1024): 32 rows
@@ -348,7 +350,13 @@ int plan_attention(fdllm_ctx* c, AttnP& a, int rows, uint16_t* kc, uint16_t* vc,
   if (sb != nullptr && !seq_kernel && !pl.chunked)
     return fail(FDLLM_EINVAL, "batched call of %d rows per sequence over %d keys is too long for one step", a.rows, a.Lk);
   a.S = pl.S; a.chunk = pl.chunk; a.target_wgs = target; a.prefill_hpw = c->prefill_hpw; a.prefill_pair = c->prefill_pair;
-  a.seq_attn = seq_kernel;
+  a.seq_attn = seq_kernel || pl.seq;
+  if (pl.seq) {
+    // rotated in place, so that out may be in fragment order; fewer splits where the allocation-free
+    // step's scratch is short
+    a.qrot = c->qkv; a.ldqr = a.ldq; a.xh = pl.xh;
+    while (t_no_alloc && a.S > 1 && attn_partial_floats(a) > c->apart_floats) --a.S;
+  }
   if (seq_kernel) {
     a.seq_cnt = c->attn_cnt;
     const size_t pf = plan_seq_units(a, c->seq_split ? c->ncu : 0);
@@ -465,6 +473,7 @@ int run_layers(fdllm_ctx* c, const void* x_in, int rows, uint16_t* kbase, uint16
       const GemmPlan pq = gemm_plan(CFG_QKV, tq, 1, c->mm);
       if (gemm_ropes_in_epilogue(CFG_QKV, pq) && g.q.ntiles % 8 == 0) {
         RopeOut& ro = g.q.ro;
+        at.qrot = nullptr;
         ro.rope = c->rope; ro.q = at.out; ro.kc = kc; ro.vc = vc;
         ro.nq = f.num_attention_heads; ro.nkv = f.num_key_value_heads;
         ro.rows = at.nseq > 1 ? at.rows : rows;
@@ -1004,10 +1013,10 @@ int fdllm_kv_write(fdllm_ctx* c, const void* k, const void* v, int rows, void* k
 
 // fast_dllm.attn_inplace (runtime.py:63-73): the write of _write_rows, then attention of the given
 // (already rotated) queries over cache rows [0, prefix_len + attend_rel) with no mask (_attend,
-// runtime.py:30-48).  The chunk and loop kernels take the queries from q (AttnP::rope null: no RoPE, and
-// ws = Lk: no rows of the call are read from q's buffer or appended, the cache already holds them); the
-// prefill kernels (128 rows and more) read rotated queries from the output buffer, where they are
-// copied first.
+// runtime.py:30-48).  The chunk kernel and attn_seq_kernel take the queries from q (AttnP::rope null: no
+// RoPE, and ws = Lk: no rows of the call are read from q's buffer or appended, the cache already holds
+// them); the prefill kernels (1024 rows and more) read rotated queries from the output buffer, where they
+// are copied first.
 int fdllm_attn_inplace(fdllm_ctx* c, const void* q, const void* k, const void* v, int rows, void* k_cache,
                        void* v_cache, int cap, int layer, int64_t prefix_len, int write_rel, int attend_rel, void* out,
                        void* stream) {
@@ -1035,7 +1044,11 @@ int fdllm_attn_inplace(fdllm_ctx* c, const void* q, const void* k, const void* v
   a.ldq = f.num_attention_heads * f.head_dim;
   a.rope = nullptr;
   a.out = (uint16_t*)out;
-  if (attn_takes_roped(a)) {
+  if (a.seq_attn) {
+    a.qrot = (uint16_t*)q;  // read only: the pass that would write them is skipped
+    a.ldqr = a.ldq;
+    a.roped = 1;
+  } else if (attn_takes_roped(a)) {
     HIPCHK(hipMemcpyAsync(out, q, (size_t)rows * a.ldq * sizeof(uint16_t), hipMemcpyDeviceToDevice, st));
     a.roped = 1;
   }

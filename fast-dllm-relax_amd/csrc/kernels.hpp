@@ -222,10 +222,15 @@ struct AttnP {
   int prefill_hpw;                    // query heads per workgroup of the prefill kernel (0: chosen per launch)
   int prefill_pair;                   // paired-query-block prefill kernel: 0 off, 1 by size, 2 always all heads per
                                       // workgroup, 3 always the heads split over workgroups
-  int seq_attn;                       // batched calls without a mask: attn_seq_kernel (no key splits) instead of chunks + merge
+  int seq_attn;                       // attn_seq_kernel: a batched call without a mask, or one sequence's (AttnPlan::seq)
   float* part;                        // split partials (merged by attn_merge_kernel)
   uint16_t* out;                      // [rows][nq * 128]
   int ofrag;                          // out in MFMA-fragment order (frag_off; rows <= 32, nseq 1)
+  // attn_seq_kernel: where the rotated queries are, [rows][ldqr] (null: in out, row-major); rope_kv_kernel
+  // writes them there (it may be qkv itself: each row's heads are rotated in place)
+  uint16_t* qrot; int ldqr;
+  int xh;                             // attn_seq_kernel, one sequence: runs of query-tile groups (AttnPlan)
+  int ncu;                            // compute units (attn_plan's splits of one sequence; 0: no attn_seq_kernel for it)
   // batched call (nseq > 1, chunked kernel only): sequence b owns rows [b rows, (b + 1) rows) of qkv,
   // rope and out, the cache at kc / vc + b seq_stride, writes from seq_ws[b] and attends
   // [0, seq_lk[b]); ws and Lk above then hold the largest window (S and chunk are planned for it)
@@ -243,8 +248,9 @@ struct AttnP {
   // launch skips rope_kv_kernel
   int roped;
 };
-struct AttnPlan { int chunked; int q_tiles_per_wg; int key_groups; int qg; int S; int chunk; };
-AttnPlan attn_plan(int rows, int nq, int nkv, int Lk, int target_wgs, int nseq);
+// seq: one sequence on attn_seq_kernel in S key splits, its query-tile groups in xh runs
+struct AttnPlan { int chunked; int q_tiles_per_wg; int key_groups; int qg; int S; int chunk; int seq; int xh; };
+AttnPlan attn_plan(int rows, int nq, int nkv, int Lk, int target_wgs, int nseq, int mask, int ncu);
 // whether launch_attention starts with rope_kv_kernel for a (the batched-sequence and prefill kernels)
 bool attn_takes_roped(const AttnP& a);
 // attn_seq_kernel's units for a batched call (a.nseq, rows, heads, seq_lk and seq_cnt set): each sequence

@@ -101,8 +101,8 @@ int fdllm_forward_cached(fdllm_ctx* ctx, const void* active_embed, int block_len
  * fdllm_forward_cached, but the step's workspace (residual stream, projections, norms, RoPE table and
  * the split partials of the projections and the attention) lives in a fixed 24 MiB device array of the
  * library, one per GPU, held until the process ends, and the call allocates and frees nothing.
- * Limits: at most 32 rows, and the attended keys must fit the scratch (the 1.5B shapes: up to 8192
- * keys through the chunked attention, more through the looped one); larger calls return FDLLM_EINVAL.
+ * Limits: at most 32 rows, and the attended keys must fit the scratch (the 1.5B shapes: up to 5120
+ * keys through the chunked attention, more through the key-streaming one, in fewer splits where short); larger calls return FDLLM_EINVAL.
  * Every call on one GPU shares that GPU's array and leaves its contents behind: calls that overlap on
  * one GPU (two streams, threads or contexts) race. */
 int fdllm_forward_cached_noalloc(fdllm_ctx* ctx, const void* active_embed, int block_len, void* k_cache,
