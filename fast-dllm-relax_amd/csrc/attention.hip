@@ -179,36 +179,25 @@ static hipError_t launch_chunk_mask(const AttnP& a, const AttnPlan& p, hipStream
   }
 }
 
-// Long row blocks: RoPE + KV append pass, then the flash-style kernel.  Two query heads per workgroup,
-// as four waves of one query tile each, once that still gives 1024 workgroups; else one head (more
-// workgroups win over fewer K/V re-reads below about that many).  Measured at 2048 and 8192 rows
-// against three heads as two waves of three tiles (one wave per SIMD either way): 38.7 against 41.4 ms
-// for the 8192-row prefill.  Three and six heads stay available through FDLLM_PREFILL_HPW.
-template <int DT, int MASK, int TQ, int NWQ>
-static hipError_t launch_prefill_cfg(const AttnP& a, int hpw, hipStream_t st) {
-  constexpr size_t lds = 2 * ((size_t)64 * (HD + 8) + (size_t)HD * (64 + 8)) * 2;
-  auto kern = attn_prefill_kernel<DT, MASK, TQ, NWQ>;
-  raise_lds(kern, lds);
-  const int nqb = (a.rows + 31) / 32, grp = a.nq / a.nkv;
-  hipLaunchKernelGGL(kern, dim3(nqb * (grp / hpw), a.nkv), dim3(64 * NWQ), lds, st, a, hpw);
-  return hipGetLastError();
-}
-
-// The paired-query-block kernel for models with 6 query heads per kv head: all heads of a kv head per
-// workgroup (PAIR_TQ tiles per wave) from PAIR_WHOLE_MIN workgroups, below that the heads split over
-// three workgroups (one tile per wave) from PAIR_SPLIT_MIN_BLOCKS query blocks, below that
-// attn_prefill_kernel; and its K/V blocks in flight.  Measured (1.5B bf16 build_prefix_cache, ms; the
-// one-block kernel / split / whole): 512 rows 3.31 / 3.38 / 3.82, 1024 4.95 / 4.89 / 5.58, 2048 8.44 /
-// 8.03 / 9.12, 4096 16.68 / 15.93 / 15.58, 8192 34.2 / 34.3 / 29.4.
-constexpr int PAIR_TQ = 3, PAIR_DEPTH = 3;
-constexpr int PAIR_WHOLE_MIN = 128, PAIR_SPLIT_MIN_BLOCKS = 32;
+// Long row blocks: the RoPE + KV append pass (unless qkv's epilogue did it), then attn_prefill_kernel, in one
+// of four forms: all of a kv head's twelve tiles per workgroup (TQ = 3, six query heads per kv head) or four,
+// query blocks paired or alone.  prefill_pair: 0 alone, 2 paired with all tiles, 3 paired with four, 1 by size:
+// four tiles alone until their workgroups pass one round of the 256 compute units by a quarter, then paired
+// (uneven blocks in a second round cost more than the pairs' fewer workgroups), all twelve alone once that
+// gives 180 workgroups and paired once the pairs give 7/8 of a round.  Measured (1.5B bf16
+// build_prefix_cache, us per layer; four alone / four paired / twelve alone / twelve paired): 509 rows 115.6 /
+// 119.3 / 123.8 / 133.4, 1500 rows 238 / 241 / 255 / 263, 2048 rows 283 / 273 / 289 / 299, 3000 rows 411 / 419 /
+// 407 / 416, 6000 rows 783 / 805 / 719 / 724, 8192 rows 1081 / 1055 / 963 / 949.
+constexpr int PREFILL_ALONE_MAX_WGS = 320, PREFILL_WHOLE_MIN_WGS = 180, PREFILL_WHOLE_PAIRED_MIN_WGS = 224;
 
 template <int DT, int MASK, int TQ>
-static hipError_t launch_pair(const AttnP& a, int pairs, int groups, hipStream_t st) {
-  auto kern = attn_prefill_pair_kernel<DT, MASK, TQ, PAIR_DEPTH>;
-  constexpr size_t lds = (size_t)(PAIR_DEPTH + 1) * 2 * 64 * HD * 2;  // K and V of D + 1 key blocks
+static hipError_t launch_prefill_cfg(const AttnP& a, int paired, hipStream_t st) {
+  auto kern = attn_prefill_kernel<DT, MASK, TQ>;
+  constexpr size_t lds = (size_t)2 * 2 * 128 * HD * 2;  // K and V of two stages of 128 keys
   raise_lds(kern, lds);
-  hipLaunchKernelGGL(kern, dim3(pairs, a.nkv, groups), dim3(256), lds, st, a);
+  const int nqb = (a.rows + 31) / 32, tiles = 2 * (a.nq / a.nkv);
+  hipLaunchKernelGGL(kern, dim3(paired ? (nqb + 1) / 2 : nqb, a.nkv, (tiles + 4 * TQ - 1) / (4 * TQ)), dim3(512), lds, st,
+                     a, paired);
   return hipGetLastError();
 }
 
@@ -216,23 +205,12 @@ template <int DT, int MASK>
 static hipError_t launch_prefill(const AttnP& a, hipStream_t st) {
   if (!a.roped) hipLaunchKernelGGL(rope_kv_kernel<DT>, dim3(a.rows), dim3(128), 0, st, a);
   const int nqb = (a.rows + 31) / 32, grp = a.nq / a.nkv;
-  const int pairs = (nqb + 1) / 2;
-  if (grp == 2 * PAIR_TQ) {
-    // prefill_pair: 0 off, 1 by size, 2 always all heads per workgroup, 3 always the split form
-    const bool whole = a.prefill_pair == 2 || (a.prefill_pair == 1 && pairs * a.nkv >= PAIR_WHOLE_MIN);
-    const bool split = a.prefill_pair == 3 || (a.prefill_pair == 1 && !whole && nqb >= PAIR_SPLIT_MIN_BLOCKS);
-    if (whole) return launch_pair<DT, MASK, PAIR_TQ>(a, pairs, 1, st);
-    if (split) return launch_pair<DT, MASK, 1>(a, pairs, PAIR_TQ, st);
+  bool paired = a.prefill_pair >= 2, whole = grp == 6 && (a.prefill_pair == 2 || a.prefill_hpw == 6);
+  if (a.prefill_pair == 1 && !whole && nqb * a.nkv * ((2 * grp + 3) / 4) > PREFILL_ALONE_MAX_WGS) {
+    whole = grp == 6 && nqb * a.nkv >= PREFILL_WHOLE_MIN_WGS;
+    paired = !whole || (nqb + 1) / 2 * a.nkv >= PREFILL_WHOLE_PAIRED_MIN_WGS;
   }
-  int hpw = grp % 2 == 0 && nqb * (grp / 2) * a.nkv >= 1024 ? 2 : 1;
-  const int ph = a.prefill_hpw;
-  if ((ph == 1 || ph == 2 || ph == 3 || ph == 6) && grp % ph == 0) hpw = ph;
-  switch (hpw) {
-    case 6: return launch_prefill_cfg<DT, MASK, 3, 4>(a, 6, st);
-    case 3: return launch_prefill_cfg<DT, MASK, 3, 2>(a, 3, st);
-    case 2: return launch_prefill_cfg<DT, MASK, 1, 4>(a, 2, st);
-    default: return launch_prefill_cfg<DT, MASK, 1, 2>(a, 1, st);
-  }
+  return whole ? launch_prefill_cfg<DT, MASK, 3>(a, paired, st) : launch_prefill_cfg<DT, MASK, 1>(a, paired, st);
 }
 
 // Batched calls without a mask: the RoPE + KV append pass over the call's rows, then attn_seq_kernel.

@@ -832,249 +832,96 @@ __global__ __launch_bounds__(128) void rope_kv_kernel(AttnP p) {
   rope_kv_row<DT>(a, (int)blockIdx.x - b * p.rows);
 }
 
-// attn_prefill_kernel: workgroup (query block of 32 rows, head subset hg of kv head g) with NWQ waves x
-// TQ query tiles (2 tiles per head: rows q0 .. q0 + 15 and q0 + 16 .. q0 + 31 of head hh).  The kv head's
-// keys stream through LDS in blocks of 64 (K row-major, V transposed), double-buffered: the next block
-// is loaded into registers while this one is multiplied, so every K/V row is read once per workgroup
-// for all of its query tiles.  Scores in fp32 on MFMA, online softmax in base 2 with the scale folded
-// in (p = 2^(s * scale * log2 e - m)), P rounded to the model dtype for P.V, fp32 accumulation; the
-// precision order of the chunk kernels.  MASK 1 (block-causal, cuda.py:148-177) reduces to a key
-// bound per query: keys below ((q_pos0 + r) / block + 1) * block.  Query blocks are dealt heaviest
-// (latest) first.  Queries come from out (rope_kv_kernel) and results go back to the same places.
-template <int DT, int MASK, int TQ, int NWQ>
-__global__ __launch_bounds__(64 * NWQ) void attn_prefill_kernel(AttnP a, int hpw) {
-  constexpr int KBP = 64;          // keys per block
-  constexpr int KLDP = HD + 8;     // u16 stride of a K row
-  constexpr int VLDP = KBP + 8;    // u16 stride of a V^T row
-  constexpr int NT = 64 * NWQ;
-  constexpr int KIT = KBP * 16 / NT;       // 16-byte K chunks per thread per block
-  constexpr int VIT = (KBP / 4) * 16 / NT; // (key quad, dim chunk) V items per thread per block
-  static_assert(KIT * NT == KBP * 16 && VIT * NT == (KBP / 4) * 16, "whole staging rounds");
-  static_assert(MASK == 0 || MASK == 1, "explicit biases take attn_kernel");
-  constexpr int DT16 = HD / 16;
-  extern __shared__ __align__(16) unsigned char smem[];
-  // buffer b: K at element b * BUFE, V^T after it.  Offsets from the shared array itself (not pointers
-  // picked from a local array), so that every access stays a direct LDS access instead of a flat one.
-  constexpr int BUFE = KBP * KLDP + HD * VLDP;
-  u16* const lds16 = reinterpret_cast<u16*>(smem);
+// One block of an online softmax over a lane's 4 N raw scores s of its query (the query's other keys sit in
+// lanes l ^ 16, l ^ 32, l ^ 48): s becomes p = 2^(s c2 - m) with m the query's reference, l the lane's part of
+// the sum of p (its four lanes' parts are added once, at the end), o the accumulator.  The reference is a
+// maximum seen so far that is renewed only when a score passes it by more than 2^LAZY_MAX: p is then at
+// most 2^8, a power of two off the usual p <= 1 and as exact (fp32, and its rounding to the model dtype,
+// are relative; fp16 holds 2^8 and loses fewer small p), and most blocks have no reduction across lanes
+// and no rescaling.  Scale and subtraction are one fma, so per score: fma, exp2, add, half a max and half a
+// rounding.
+constexpr float LAZY_MAX = 8.0f;
 
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int lr = lane & 15, lg = lane >> 4;
-  const int grp = a.nq / a.nkv, nhg = grp / hpw;
-  const int nqb = (a.rows + 31) / 32;
-  const int qb = nqb - 1 - (int)blockIdx.x / nhg, hg = (int)blockIdx.x % nhg;
-  const int g = blockIdx.y;
-  const int q0 = qb * 32, rlast = a.rows - 1;
-  const size_t krow = (size_t)a.nkv * HD;
-  const u16* kc = a.kc + g * HD;
-  const u16* vc = a.vc + g * HD;
-  const float c2 = a.scale * LOG2E;
-
-  // the keys this workgroup needs: up to its last query's bound
-  auto kend_of = [&](int r) {
-    if constexpr (MASK == 1) return min(a.Lk, ((a.q_pos0 + r) / a.block + 1) * a.block);
-    return a.Lk;
-  };
-  const int kend_wg = kend_of(min(q0 + 31, rlast));
-  const int nkb = (kend_wg + KBP - 1) / KBP;
-
-  // this wave's query tiles: tile t = w TQ + i -> head hg hpw + t / 2, rows q0 + 16 (t % 2) + lr
-  u32x4 qf[TQ][4];
-  int kend_q[TQ];
-  bool tvalid[TQ];
-  const u16* qsrc = a.out;
+// two probabilities rounded to the model dtype: 2^x is no product, so fp16 needs none of pack_f32x2's care
+// about mixed-precision fmas (whose empty asm keeps the values in registers of their own)
+template <int DT> __device__ __forceinline__ uint32_t pack_p(float a, float b) {
+  if constexpr (DT == DT_BF16) return pack_f32x2<DT>(a, b);
+  else return pack2(f32_to_f16(a), f32_to_f16(b));
+}
+template <int N, int NO>
+__device__ __forceinline__ void lazy_softmax(f32x4 (&s)[N], float c2, float& m, float& l, f32x4 (&o)[NO]) {
+  float mx = s[0][0];
 #pragma unroll
-  for (int i = 0; i < TQ; ++i) {
-    const int t = w * TQ + i;
-    tvalid[i] = t < 2 * hpw && q0 + 16 * (t % 2) <= rlast;
-    const int hh = hg * hpw + min(t, 2 * hpw - 1) / 2;
-    const int r = min(q0 + 16 * (t % 2) + lr, rlast);
-    kend_q[i] = kend_of(r);
-    const u16* qp = qsrc + (size_t)r * a.nq * HD + (g * grp + hh) * HD + 8 * lg;
+  for (int kt = 0; kt < N; ++kt)
 #pragma unroll
-    for (int ds = 0; ds < 4; ++ds) qf[i][ds] = *reinterpret_cast<const u32x4*>(qp + 32 * ds);
+    for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[kt][e]);
+  mx *= c2;
+  if (__builtin_amdgcn_ballot_w64(mx > m + LAZY_MAX) != 0) {
+    const float m_new = fmaxf(m, rows_max(mx));
+    const float alpha = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.f : m_new));
+    l *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < NO; ++dt) o[dt] *= alpha;
+    m = m_new;
   }
-
-  // staging maps (conflict-free LDS stores): K item -> key j, 16-byte chunk c; V item -> key quad kq, dim chunk dc
-  u32x4 kr[KIT], vr[VIT][4];
-  auto load = [&](int kb) {
-    const int k0 = kb * KBP;
+  const float nm = m == -INFINITY ? 0.f : -m;
 #pragma unroll
-    for (int it = 0; it < KIT; ++it) {
-      const int item = threadIdx.x + it * NT;
-      const int j = (item & 15) + 16 * (item >> 8), c = (item >> 4) & 15;
-      const int key = min(k0 + j, kend_wg - 1);
-      kr[it] = *reinterpret_cast<const u32x4*>(kc + (size_t)key * krow + 8 * c);
+  for (int kt = 0; kt < N; ++kt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[kt][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][e], c2, nm));
+      l += s[kt][e];
     }
-#pragma unroll
-    for (int it = 0; it < VIT; ++it) {
-      const int item = threadIdx.x + it * NT;
-      const int kq = item & 15, dc = item >> 4;
-#pragma unroll
-      for (int qq = 0; qq < 4; ++qq) {
-        const int key = min(k0 + 4 * kq + qq, kend_wg - 1);
-        vr[it][qq] = *reinterpret_cast<const u32x4*>(vc + (size_t)key * krow + 8 * dc);
-      }
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int it = 0; it < KIT; ++it) {
-      const int item = threadIdx.x + it * NT;
-      const int j = (item & 15) + 16 * (item >> 8), c = (item >> 4) & 15;
-      *reinterpret_cast<u32x4*>(lds16 + buf * BUFE + j * KLDP + 8 * c) = kr[it];
-    }
-#pragma unroll
-    for (int it = 0; it < VIT; ++it) {
-      const int item = threadIdx.x + it * NT;
-      const int kq = item & 15, dc = item >> 4;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
-        const uint32_t w01 = __builtin_amdgcn_perm(vr[it][1][e >> 1], vr[it][0][e >> 1], sel);
-        const uint32_t w23 = __builtin_amdgcn_perm(vr[it][3][e >> 1], vr[it][2][e >> 1], sel);
-        *reinterpret_cast<u32x2*>(lds16 + buf * BUFE + KBP * KLDP + (8 * dc + e) * VLDP + 4 * kq) = u32x2{w01, w23};
-      }
-    }
-  };
-
-  float m_run[TQ], l_run[TQ];
-  f32x4 o[TQ][DT16];
-#pragma unroll
-  for (int i = 0; i < TQ; ++i) {
-    m_run[i] = -INFINITY;
-    l_run[i] = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < DT16; ++dt) o[i][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-
-  load(0);
-  stage(0);
-  __syncthreads();
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int buf = kb & 1;
-    load(min(kb + 1, nkb - 1));
-    const u16* kbuf = lds16 + buf * BUFE;
-    const u16* vbuf = kbuf + KBP * KLDP;
-    const int k0 = kb * KBP;
-#pragma unroll
-    for (int i = 0; i < TQ; ++i) {
-      if (!tvalid[i]) continue;
-      // S^T = K Q^T: lane holds S^T[key k0 + 16 kt + 4 lg + e][query lr]
-      f32x4 s[4];
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
-        s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const u16* kp = kbuf + (16 * kt + lr) * KLDP + 8 * lg;
-#pragma unroll
-        for (int ds = 0; ds < 4; ++ds) s[kt] = mfma16<DT>(*reinterpret_cast<const u32x4*>(kp + 32 * ds), qf[i][ds], s[kt]);
-      }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int key = k0 + 16 * kt + 4 * lg + e;
-          const float v = key < kend_q[i] ? s[kt][e] * c2 : -INFINITY;
-          s[kt][e] = v;
-          mx = fmaxf(mx, v);
-        }
-      mx = rows_max(mx);
-      const float m_new = fmaxf(m_run[i], mx);
-      const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m_run[i] - m_use);
-      float ps = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float pe = __builtin_amdgcn_exp2f(s[kt][e] - m_use);
-          s[kt][e] = pe;
-          ps += pe;
-        }
-      ps = rows_sum(ps);
-      l_run[i] = l_run[i] * alpha + ps;
-      m_run[i] = m_new;
-#pragma unroll
-      for (int dt = 0; dt < DT16; ++dt) o[i][dt] *= alpha;
-      // O^T += V^T P^T over the block's two 32-key k steps (k slot 8 lg + e: key 4 lg + e, then 16 + 4 lg + e - 4)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const u32x4 pb = {pack2(from_f32<DT>(s[2 * ks][0]), from_f32<DT>(s[2 * ks][1])),
-                          pack2(from_f32<DT>(s[2 * ks][2]), from_f32<DT>(s[2 * ks][3])),
-                          pack2(from_f32<DT>(s[2 * ks + 1][0]), from_f32<DT>(s[2 * ks + 1][1])),
-                          pack2(from_f32<DT>(s[2 * ks + 1][2]), from_f32<DT>(s[2 * ks + 1][3]))};
-#pragma unroll
-        for (int dt = 0; dt < DT16; ++dt) {
-          const u16* vrow = vbuf + (16 * dt + lr) * VLDP + 32 * ks + 4 * lg;
-          const u32x2 lo = *reinterpret_cast<const u32x2*>(vrow);
-          const u32x2 hi = *reinterpret_cast<const u32x2*>(vrow + 16);
-          o[i][dt] = mfma16<DT>(u32x4{lo[0], lo[1], hi[0], hi[1]}, pb, o[i][dt]);
-        }
-      }
-    }
-    stage(buf ^ 1);
-    __syncthreads();
-  }
-
-  // lane output: query row r of tile i, dims 16 dt + 4 lg .. + 3
-#pragma unroll
-  for (int i = 0; i < TQ; ++i) {
-    const int t = w * TQ + i;
-    const int r = q0 + 16 * (t % 2) + lr;
-    if (!tvalid[i] || r > rlast) continue;
-    const int hh = hg * hpw + t / 2;
-    const float inv = 1.0f / l_run[i];
-    u16* dst = a.out + (size_t)r * a.nq * HD + (g * grp + hh) * HD + 4 * lg;
-#pragma unroll
-    for (int dt = 0; dt < DT16; ++dt)
-      *reinterpret_cast<u32x2*>(dst + 16 * dt) =
-          u32x2{pack2(from_f32<DT>(o[i][dt][0] * inv), from_f32<DT>(o[i][dt][1] * inv)),
-                pack2(from_f32<DT>(o[i][dt][2] * inv), from_f32<DT>(o[i][dt][3] * inv))};
-  }
 }
 
-// attn_prefill_pair_kernel: the long-prefill form of attn_prefill_kernel.  Workgroup (p, g) owns kv head
-// g and the pair of 32-row query blocks nqb - 1 - p and p: under the block-causal mask their key ranges
-// add up to the same number of 64-key blocks for every pair, so with one workgroup per compute unit all
-// finish together (one block per workgroup, as in attn_prefill_kernel, leaves the longest query block
-// alone on its compute unit at the end).  The workgroup's 4 TQ query tiles (TQ per wave) are tiles
-// 4 TQ z .. of the kv head's 2 grp (blockIdx.z = z): with TQ = grp / 2 all heads of the kv head are in one
-// workgroup, so each K/V block fetched serves all of them; shorter prefills, with too few pairs to fill
-// the chip, split the heads over 2 grp / (4 TQ) workgroups.  A wave reads each K or V fragment from LDS
-// once for its TQ tiles.  Per query the key blocks, their order and every rounding are
-// those of attn_prefill_kernel, so the results are the same bits.
+// attn_prefill_kernel: workgroup (x, g, z) owns 32-row query blocks of kv head g: with `paired` the blocks
+// nqb - 1 - x and x (under the block-causal mask every pair has the same number of key blocks, so with one
+// workgroup per compute unit all finish together), else block nqb - 1 - x alone (the heaviest first; short
+// prefills, whose pairs would leave compute units idle).  Of the kv head's 2 grp query tiles (rows q0 .. + 15
+// and q0 + 16 .. + 31 of each head) it takes 4 TQ from 4 TQ z: TQ = 3 is all twelve of a kv head with six
+// heads, so each K/V block fetched serves all of them; TQ = 1 spreads the heads over workgroups.
 //
-// The work is a list of tasks t = (query block, key block): the first block's key blocks, then the
-// second's.  Task t's K and V rows go from global memory straight into LDS buffer t % R (R = D + 1) by
-// the gfx950 global-to-LDS copy, D tasks ahead, so no registers hold data in flight and no VALU work
-// stages it.  Both are stored row-major (a 256-byte row per key) with the 16-byte chunk c of row r at
-// slot c ^ (r % 16): the copy's lanes fetch their chunks in that order, the K fragment reads (16 rows,
-// one chunk each) then hit 16 different slots, and so do the V reads.  V^T fragments come from the
-// transposing LDS read (ds_read_b64_tr_b16): within each 16-lane group, lane q supplies 4 dims of one
-// key (key q / 4, dims 4 (q % 4) ..) and lane m receives dim m of the 4 keys, which is the A operand of
-// O^T = V^T P^T for keys 4 lg .. 4 lg + 3 (and, from a second read, 16 + 4 lg ..): the k-slot order the
-// scores already have in registers.
-template <int DT, int MASK, int TQ, int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void attn_prefill_pair_kernel(AttnP a) {
-  constexpr int NWQ = 4, R = D + 1;
-  constexpr int KBP = 64;               // keys per block (task)
-  constexpr int BUFE = 2 * KBP * HD;    // u16 per buffer: K rows, then V rows
-  constexpr int CPW = KBP * HD * 2 / 1024 / NWQ;  // 1 KB copies of K (and of V) per wave per task
+// Eight waves: wave w takes tiles 4 TQ z + (w % 4) TQ .. + TQ - 1 and key part kh = w / 4, the first or the
+// second 64 keys of every 128-key stage.  Two waves per SIMD, so that one's softmax (VALU) runs while the
+// other's MFMAs do: with four waves and no key parts a stage's MFMAs (1536 cycles of a SIMD), softmax
+// (about 1900) and LDS waits followed one another (per layer at 8192 / 2048 / 509 rows: 317 / 50 / 14.4 us with
+// one wave per SIMD, 277 / 41.6 us with lazy_softmax as well, 212 / 35 / 10.7 us with both; 1.0 PFLOP/s at 8192).
+// The parts of a query block are merged through LDS when its keys end (part 0 + part 1, each relative to the
+// larger maximum).  MFMAs and VALU work now bound it, about equally.
+//
+// The work is a list of stages t = (query block, 128 keys): the first block's, then the second's.  Stage
+// t's K and V rows go from global memory straight into LDS buffer t % 2 by the gfx950 global-to-LDS copy, a
+// stage ahead, so no registers hold data in flight and no VALU work stages it.  Both are stored row-major (a
+// 256-byte row per key) with the 16-byte chunk c of row r at slot c ^ (r % 16): the copy's lanes fetch their
+// chunks in that order, the K fragment reads (16 rows, one chunk each) then hit 16 different slots, and so
+// do the V reads.  V^T fragments come from the transposing LDS read (ds_read_b64_tr_b16): within each 16-lane
+// group, lane q supplies 4 dims of one key (key q / 4, dims 4 (q % 4) ..) and lane m receives dim m of the 4
+// keys, which is the A operand of O^T = V^T P^T for keys 4 lg .. 4 lg + 3 (and, from a second read, 16 + 4
+// lg ..): the k-slot order the scores already have in registers.
+//
+// MASK 1 (block-causal, cuda.py:148-177) reduces to a key bound per query: keys below ((q_pos0 + r) / block
+// + 1) * block.  Queries come from out (rope_kv_kernel, or qkv's epilogue) and results go back to the same
+// places.  A query's arithmetic does not depend on TQ or on the pairing: every form gives the same bits.
+template <int DT, int MASK, int TQ>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void attn_prefill_kernel(AttnP a, int paired) {
+  constexpr int NWQ = 4, KHP = 2;                  // tile slots, key parts
+  constexpr int KBP = 64, STK = KHP * KBP;         // keys per part and per stage
+  constexpr int BUFB = 2 * STK * HD * 2;           // bytes per buffer: K rows, then V rows
+  constexpr int CPW = STK * HD * 2 / 1024 / (NWQ * KHP);  // 1 KB copies of K (and of V) per wave per stage
   static_assert(MASK == 0 || MASK == 1, "explicit biases take attn_kernel");
-  static_assert(D >= 1 && (D - 1) * 2 * CPW < 64, "outstanding copies fit the memory counter");
   constexpr int DT16 = HD / 16;
+  static_assert(NWQ * DT16 * 1024 + NWQ * 128 <= BUFB, "a round of the part merge fits one buffer");
   extern __shared__ __align__(16) unsigned char smem[];
-  u16* const lds16 = reinterpret_cast<u16*>(smem);
 
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wq = w % NWQ, kh = w / NWQ;
   const int lr = lane & 15, lg = lane >> 4;
-  const int grp = a.nq / a.nkv;  // = NWQ TQ gridDim.z / 2 (the launcher checks)
+  const int grp = a.nq / a.nkv;
   const int nqb = (a.rows + 31) / 32;
-  const int p = blockIdx.x, g = blockIdx.y;
-  const int tq0 = (int)blockIdx.z * NWQ * TQ;  // the workgroup's first query tile of the kv head
-  const int qA = nqb - 1 - p, qB = p;  // qA == qB: the middle block of an odd count, alone
+  const int g = blockIdx.y;
+  const int tq0 = (int)blockIdx.z * NWQ * TQ + wq * TQ;  // the wave's first query tile of the kv head
+  const int qA = nqb - 1 - (int)blockIdx.x, qB = paired ? (int)blockIdx.x : qA;  // equal: one block alone
   const int rlast = a.rows - 1;
   const size_t krow = (size_t)a.nkv * HD;
   const u16* kc = a.kc + g * HD;
@@ -1087,33 +934,47 @@ void attn_prefill_pair_kernel(AttnP a) {
   };
   auto kend_blk = [&](int qb) { return kend_of(min(qb * 32 + 31, rlast)); };
   const int keA = kend_blk(qA), keB = kend_blk(qB);
-  const int nA = (keA + KBP - 1) / KBP;
-  // this lane's K fragment byte offsets within a buffer: row lr, chunk lg + 4 ds (swizzled; + 4096 bytes
-  // per 16-row score tile)
-  uint32_t koff[4];
-#pragma unroll
-  for (int ds = 0; ds < 4; ++ds) koff[ds] = 2 * (lr * HD + 8 * ((lg + 4 * ds) ^ lr));
-  const int T = nA + (qA == qB ? 0 : (keB + KBP - 1) / KBP);
+  const int nA = (keA + STK - 1) / STK;
+  const int T = nA + (qA == qB ? 0 : (keB + STK - 1) / STK);
+  // this lane's K fragment byte offset within a buffer: row 64 kh + lr, chunk lg (swizzled); chunk lg + 4 ds is
+  // koff ^ 64 ds (a row is 256 bytes and 4 ds flips bits 2 and 3 of the chunk), + 4096 bytes per 16-row score
+  // tile.  Its V^T read offset: key 64 kh + 4 lg + lr / 4, dims 4 (lr % 4) .. + 3; dims 16 dt + .. at voff ^
+  // 32 dt, + 4096 bytes for the second half of a 32-key step, + 8192 per step.  (One register each: the
+  // offsets kept for every ds and dt spilled.)
+  const uint32_t koff = 2 * ((KBP * kh + lr) * HD + 8 * (lg ^ lr));
+  const uint32_t voff = 2 * ((STK + KBP * kh + 4 * lg + (lr >> 2)) * HD +
+                             8 * (((lr & 3) >> 1) ^ (4 * lg + (lr >> 2))) + 4 * (lr & 1));
 
-  // ---- copies of task t (tasks past the last re-read the last) into buffer t % R: this wave's 1 KB
-  // blocks d = w CPW .. + CPW - 1 of K and of V, 4 rows each; lane l fills row 4 d + l / 16, slot l % 16
-  // with chunk (l % 16) ^ (row % 16) ----
+  // ---- copies of stage t into buffer t % 2: this wave's 1 KB blocks d = w CPW .. + CPW - 1 of K and of V,
+  // 4 rows each; lane l fills row 4 d + l / 16, slot l % 16 with chunk (l % 16) ^ (row % 16) ----
+  static_assert(CPW == 4, "a wave's rows start at a multiple of 16");
+  // the lane's source for c = 0 (row 16 w + lane / 16); row + 4 c adds 4 c rows and flips bits 2 and 3 of the chunk
+  const int src0 = (4 * CPW * w + (lane >> 4)) * (int)krow + 8 * ((lane & 15) ^ (lane >> 4));
   auto issue = [&](int t) __attribute__((always_inline)) {
-    const int tt = min(t, T - 1);
-    const int k0 = (tt < nA ? tt : tt - nA) * KBP, kend = tt < nA ? keA : keB;
-    unsigned char* buf = smem + (size_t)(t % R) * BUFE * 2;
+    const int k0 = (t < nA ? t : t - nA) * STK, kend = t < nA ? keA : keB;
+    unsigned char* buf = smem + (size_t)(t & 1) * BUFB;
+    const u16* kb = kc + (size_t)k0 * krow;
+    const u16* vb = vc + (size_t)k0 * krow;
+    if (k0 + STK <= kend) {
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      const int d = w * CPW + c, row = 4 * d + (lane >> 4);
-      const int chunk = (lane & 15) ^ (row & 15);
-      const size_t src = (size_t)min(k0 + row, kend - 1) * krow + 8 * chunk;
-      lds_copy16(kc + src, buf + (size_t)d * 1024);
-      lds_copy16(vc + src, buf + (size_t)KBP * HD * 2 + (size_t)d * 1024);
+      for (int c = 0; c < CPW; ++c) {
+        const int d = w * CPW + c, src = src0 ^ (32 * c);
+        lds_copy16(kb + (size_t)(4 * c) * krow + src, buf + (size_t)d * 1024);
+        lds_copy16(vb + (size_t)(4 * c) * krow + src, buf + (size_t)STK * HD * 2 + (size_t)d * 1024);
+      }
+    } else {  // rows past the last key repeat it (masked)
+#pragma unroll
+      for (int c = 0; c < CPW; ++c) {
+        const int d = w * CPW + c, row = 4 * d + (lane >> 4);
+        const int src = (min(k0 + row, kend - 1) - k0) * (int)krow + 8 * ((lane & 15) ^ (row & 15));
+        lds_copy16(kb + src, buf + (size_t)d * 1024);
+        lds_copy16(vb + src, buf + (size_t)STK * HD * 2 + (size_t)d * 1024);
+      }
     }
   };
 
-  // ---- the wave's query tiles of the current query block: tile w TQ + i = head (w TQ + i) / 2, rows
-  // q0 + 16 ((w TQ + i) % 2) + lr ----
+  // ---- the wave's query tiles of the current query block: tile t = tq0 + i is head t / 2, rows q0 + 16 (t %
+  // 2) + lr (tiles past the kv head's 2 grp repeat the last and store nothing) ----
   u32x4 qf[TQ][4];
   int kend_q[TQ];
   int kend_min = 0;  // the block's first row's key bound, the smallest of its rows
@@ -1121,197 +982,167 @@ void attn_prefill_pair_kernel(AttnP a) {
   f32x4 o[TQ][DT16];
   auto begin_block = [&](int qb) __attribute__((always_inline)) {
     const int q0 = qb * 32;
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // (here and in end_block: the addresses are formed here, not kept through the loop)
+    const int lrb = ln & 15, lgb = ln >> 4;
     kend_min = kend_of(q0);
 #pragma unroll
     for (int i = 0; i < TQ; ++i) {
-      const int t = tq0 + w * TQ + i, hh = t / 2;
-      const int r = min(q0 + 16 * (t % 2) + lr, rlast);
+      const int t = min(tq0 + i, 2 * grp - 1), hh = t / 2;
+      const int r = min(q0 + 16 * (t % 2) + lrb, rlast);
       kend_q[i] = kend_of(r);
-      const u16* qp = a.out + (size_t)r * a.nq * HD + (g * grp + hh) * HD + 8 * lg;
+      const u16* qp = a.out + (size_t)r * a.nq * HD + (g * grp + hh) * HD + 8 * lgb;
 #pragma unroll
       for (int ds = 0; ds < 4; ++ds) qf[i][ds] = *reinterpret_cast<const u32x4*>(qp + 32 * ds);
-      // o is not cleared here: with m_run = -inf the block's first key block rescales it by
-      // alpha = 2^-inf = 0 (o is always finite, and -0 + x = x)
       m_run[i] = -INFINITY;
       l_run[i] = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < DT16; ++dt) o[i][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    // the query loads land here, once per query block: otherwise the compiler's wait before the first
-    // MFMA of every key block covers them (they may be the youngest loads on the other path of the
-    // branch), which waits for every copy in flight and drains the copy pipeline on each block
+    // the query loads land here, once per query block (left outstanding, the compiler's wait before the
+    // first MFMA of every stage would cover them, and with them the copies in flight)
     wait_vmcnt<0>();
   };
-  auto end_block = [&](int qb) __attribute__((always_inline)) {
+  // the parts' merge and the block's output; buffer t % 2 (stage t's, read by every wave once they meet here)
+  // holds one tile of each of the four slots at a time
+  auto end_block = [&](int qb, int t) __attribute__((always_inline)) {
     const int q0 = qb * 32;
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int lrb = ln & 15, lgb = ln >> 4;
+    f32x4* xo = reinterpret_cast<f32x4*>(smem + (size_t)(t & 1) * BUFB) + wq * DT16 * 64 + ln;
+    float* xm = reinterpret_cast<float*>(smem + (size_t)(t & 1) * BUFB + NWQ * DT16 * 1024) + wq * 32 + lrb;
 #pragma unroll
     for (int i = 0; i < TQ; ++i) {
-      const int t = tq0 + w * TQ + i, hh = t / 2;
-      const int r = q0 + 16 * (t % 2) + lr;
-      if (r > rlast) continue;
-      const float inv = 1.0f / l_run[i];
-      u16* dst = a.out + (size_t)r * a.nq * HD + (g * grp + hh) * HD + 4 * lg;
+      const float l = rows_sum(l_run[i]);
+      __syncthreads();
+      if (kh == 1) {
 #pragma unroll
-      for (int dt = 0; dt < DT16; ++dt)
-        *reinterpret_cast<u32x2*>(dst + 16 * dt) =
-            u32x2{pack_f32x2<DT>(o[i][dt][0] * inv, o[i][dt][1] * inv), pack_f32x2<DT>(o[i][dt][2] * inv, o[i][dt][3] * inv)};
+        for (int dt = 0; dt < DT16; ++dt) xo[dt * 64] = o[i][dt];
+        if (lgb == 0) {
+          xm[0] = m_run[i];
+          xm[16] = l;
+        }
+      }
+      __syncthreads();
+      if (kh == 0) {
+        const float m1 = xm[0], M = fmaxf(m_run[i], m1), Mu = M == -INFINITY ? 0.f : M;
+        const float f0 = __builtin_amdgcn_exp2f(m_run[i] - Mu), f1 = __builtin_amdgcn_exp2f(m1 - Mu);
+        const float inv = 1.0f / (l * f0 + xm[16] * f1);
+        const int tt = tq0 + i, hh = tt / 2, r = q0 + 16 * (tt % 2) + lrb;
+        if (tt < 2 * grp && r <= rlast) {
+          u16* dst = a.out + (size_t)r * a.nq * HD + (g * grp + hh) * HD + 4 * lgb;
+#pragma unroll
+          for (int dt = 0; dt < DT16; ++dt) {
+            const f32x4 v = o[i][dt] * f0 + xo[dt * 64] * f1;
+            *reinterpret_cast<u32x2*>(dst + 16 * dt) =
+                u32x2{pack_f32x2<DT>(v[0] * inv, v[1] * inv), pack_f32x2<DT>(v[2] * inv, v[3] * inv)};
+          }
+        }
+      }
     }
   };
 
-  // ---- one key block of task t against the wave's TQ tiles ----
+  // ---- the wave's part of stage t against its TQ tiles ----
+  const uint32_t lds0 = lds_addr(smem);
   auto compute = [&](int t) __attribute__((always_inline)) {
-    const u16* kbuf = lds16 + (size_t)(t % R) * BUFE;
-    const u16* vbuf = kbuf + KBP * HD;
-    const int k0 = (t < nA ? t : t - nA) * KBP;
-    // S^T = K Q^T: lane holds S^T[key k0 + 16 kt + 4 lg + e][query lr]; K row 16 kt + lr, chunk lg + 4 ds.
-    // The four fragments of score tile kt + 1 are requested (asm reads, one wait for the four) before tile
-    // kt's MFMAs, so each wait finds them landed (the compiler's own order read one fragment, waited the
-    // whole LDS latency and issued its TQ MFMAs, sixteen times per block)
+    const uint32_t ka = lds0 + (uint32_t)(t & 1) * BUFB + koff, va0 = lds0 + (uint32_t)(t & 1) * BUFB + voff;
+    const int k0 = (t < nA ? t : t - nA) * STK + KBP * kh;  // the part's first key
+    // S^T = K Q^T: lane holds S^T[key k0 + 16 kt + 4 lg + e][query lr].  K fragments two at a time, the next two
+    // requested (asm reads, one wait for both) before these two's MFMAs
     f32x4 s[TQ][4];
-    const uint32_t kbb = lds_addr(kbuf);
-    u32x4 kf0[4], kf1[4];
-    auto rdk = [&](auto ktc, u32x4 (&f)[4]) __attribute__((always_inline)) {
-      constexpr int KT = decltype(ktc)::value;
+    u32x4 kf[2][2];
+    static_for<0, 9>([&](auto hc) __attribute__((always_inline)) {
+      constexpr int H = decltype(hc)::value;  // half H: score tile H / 2, fragments 2 (H % 2) and the next
+      if constexpr (H < 8) {
 #pragma unroll
-      for (int ds = 0; ds < 4; ++ds) f[ds] = ds_read16<KT * 4096>(kbb + koff[ds]);
-    };
-    auto mmk = [&](int kt, const u32x4 (&f)[4]) __attribute__((always_inline)) {
+        for (int d = 0; d < 2; ++d) kf[H & 1][d] = ds_read16<(H >> 1) * 4096>(ka ^ (64 * (2 * (H & 1) + d)));
+      }
+      if constexpr (H > 0) {
+        constexpr int G = H - 1, kt = G >> 1;
+        if constexpr ((G & 1) == 0) {
 #pragma unroll
-      for (int i = 0; i < TQ; ++i) s[i][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ds = 0; ds < 4; ++ds)
-#pragma unroll
-        for (int i = 0; i < TQ; ++i) s[i][kt] = mfma16<DT>(f[ds], qf[i][ds], s[i][kt]);
-    };
-    rdk(std::integral_constant<int, 0>{}, kf0);
-    lds_wait(kf0);
-    rdk(std::integral_constant<int, 1>{}, kf1);
-    mmk(0, kf0);
-    lds_wait(kf1);
-    rdk(std::integral_constant<int, 2>{}, kf0);
-    mmk(1, kf1);
-    lds_wait(kf0);
-    rdk(std::integral_constant<int, 3>{}, kf1);
-    mmk(2, kf0);
-    lds_wait(kf1);
-    mmk(3, kf1);
-    // V^T fragments of k step ks by transposing reads (ds_read_tr16: the builtin would make the compiler
-    // wait for every copy in flight first): this lane supplies key 32 ks + 4 lg + lr / 4 (+ 16 for the
-    // second half), dims 16 dt + 4 (lr % 4) .. + 3.  k step 0's reads are issued here and land during the
-    // softmax; k step 1's during k step 0's MFMAs (both k steps' P.V after each tile's own softmax
-    // measured the same, with 30 more registers)
-    const uint32_t vbase = lds_addr(vbuf);
-    auto rdv = [&](int ks, u32x2 (&vh)[DT16 * 2]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int dt = 0; dt < DT16; ++dt)
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-          const int row = 32 * ks + 16 * hf + 4 * lg + (lr >> 2);
-          const int dim = 16 * dt + 4 * (lr & 3);
-          vh[dt * 2 + hf] = ds_read_tr16(vbase + 2 * (row * HD + 8 * ((dim >> 3) ^ (row & 15)) + (dim & 7)));
+          for (int i = 0; i < TQ; ++i) s[i][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+#pragma unroll
+          for (int i = 0; i < TQ; ++i) s[i][kt] = mfma16<DT>(kf[G & 1][d], qf[i][2 * (G & 1) + d], s[i][kt]);
+      }
+      if constexpr (H < 8) lds_wait(kf[H & 1]);
+    });
+    // V^T fragments of 32-key step ks, four dim tiles at a time
+    auto rdv = [&](auto ksc, auto hc, u32x2 (&vh)[DT16]) __attribute__((always_inline)) {
+      constexpr int KSI = decltype(ksc)::value, H = decltype(hc)::value;
+#pragma unroll
+      for (int dt = 0; dt < DT16 / 2; ++dt) {
+        const uint32_t va = va0 ^ (32 * (H * DT16 / 2 + dt));
+        vh[dt * 2] = ds_read_tr16<KSI * 8192>(va);
+        vh[dt * 2 + 1] = ds_read_tr16<KSI * 8192 + 4096>(va);
+      }
     };
-    u32x2 vh0[DT16 * 2], vh1[DT16 * 2];
-    rdv(0, vh0);
+    u32x2 va[DT16], vb[DT16];
+    rdv(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, va);  // lands during the softmax
     u32x4 pb[TQ][2];
-    const bool whole = k0 + KBP <= kend_min;  // no key of the block is masked for any query of the block
+    const bool whole = k0 + KBP <= kend_min;  // no key of the part is masked for any query of the block
 #pragma unroll
     for (int i = 0; i < TQ; ++i) {
-      float mx = -INFINITY;
-      if (whole) {
+      if (!whole) {
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            s[i][kt][e] *= c2;
-            mx = fmaxf(mx, s[i][kt][e]);
-          }
-      } else {
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int key = k0 + 16 * kt + 4 * lg + e;
-            const float v = key < kend_q[i] ? s[i][kt][e] * c2 : -INFINITY;
-            s[i][kt][e] = v;
-            mx = fmaxf(mx, v);
-          }
+          for (int e = 0; e < 4; ++e)
+            s[i][kt][e] = k0 + 16 * kt + 4 * lg + e < kend_q[i] ? s[i][kt][e] : -INFINITY;
       }
-      mx = rows_max(mx);
-      const float m_new = fmaxf(m_run[i], mx);
-      const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m_run[i] - m_use);
-      float ps = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float pe = __builtin_amdgcn_exp2f(s[i][kt][e] - m_use);
-          s[i][kt][e] = pe;
-          ps += pe;
-        }
-      ps = rows_sum(ps);
-      l_run[i] = l_run[i] * alpha + ps;
-      m_run[i] = m_new;
-      // rescale only when some query's running maximum moved (alpha = 1 leaves o unchanged bit for bit);
-      // past the first blocks it rarely does, and o can stay in the accumulation registers
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-        for (int dt = 0; dt < DT16; ++dt) o[i][dt] *= alpha;
-      }
+      lazy_softmax(s[i], c2, m_run[i], l_run[i], o[i]);
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
-        pb[i][ks] = u32x4{pack_f32x2<DT>(s[i][2 * ks][0], s[i][2 * ks][1]),
-                          pack_f32x2<DT>(s[i][2 * ks][2], s[i][2 * ks][3]),
-                          pack_f32x2<DT>(s[i][2 * ks + 1][0], s[i][2 * ks + 1][1]),
-                          pack_f32x2<DT>(s[i][2 * ks + 1][2], s[i][2 * ks + 1][3])};
+        pb[i][ks] = u32x4{pack_p<DT>(s[i][2 * ks][0], s[i][2 * ks][1]),
+                          pack_p<DT>(s[i][2 * ks][2], s[i][2 * ks][3]),
+                          pack_p<DT>(s[i][2 * ks + 1][0], s[i][2 * ks + 1][1]),
+                          pack_p<DT>(s[i][2 * ks + 1][2], s[i][2 * ks + 1][3])};
     }
-    // O^T += V^T P^T over the block's two 32-key k steps
-    auto mmv = [&](int ks, const u32x2 (&vh)[DT16 * 2]) __attribute__((always_inline)) {
+    // O^T += V^T P^T over the part's two 32-key steps
+    auto mmv = [&](int ks, int h, const u32x2 (&vh)[DT16]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int dt = 0; dt < DT16; ++dt) {
+      for (int dt = 0; dt < DT16 / 2; ++dt) {
         const u32x4 vf = u32x4{vh[2 * dt][0], vh[2 * dt][1], vh[2 * dt + 1][0], vh[2 * dt + 1][1]};
 #pragma unroll
-        for (int i = 0; i < TQ; ++i) o[i][dt] = mfma16<DT>(vf, pb[i][ks], o[i][dt]);
+        for (int i = 0; i < TQ; ++i) o[i][h * DT16 / 2 + dt] = mfma16<DT>(vf, pb[i][ks], o[i][h * DT16 / 2 + dt]);
       }
     };
-    lds_wait(vh0);
-    rdv(1, vh1);
-    mmv(0, vh0);
-    lds_wait(vh1);
-    mmv(1, vh1);
+    lds_wait(va);
+    rdv(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, vb);
+    mmv(0, 0, va);
+    lds_wait(vb);
+    rdv(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}, va);
+    mmv(0, 1, vb);
+    lds_wait(va);
+    rdv(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, vb);
+    mmv(1, 0, va);
+    lds_wait(vb);
+    mmv(1, 1, vb);
   };
 
-  // ---- task t: wait for its copies, free buffer (t - 1) % R, issue task t + D into it, compute.
-  // EXACT: the D - 1 tasks issued after task t each issued 2 CPW copies per wave, so a count wait is
-  // exact (loads and stores of queries and outputs issued in between only make it wait longer); the last
-  // T % D tasks, after the loop, wait for everything ----
-  auto iter = [&](int t, auto exact) __attribute__((always_inline)) {
-    if constexpr (decltype(exact)::value) wait_vmcnt<(D - 1) * 2 * CPW>();
-    else wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();  // every wave's copies of task t have landed; buffer (t - 1) % R is free
-    __builtin_amdgcn_sched_barrier(0);
-    issue(t + D);
-    __builtin_amdgcn_sched_barrier(0);
-    if (t == nA) begin_block(qB);
-    compute(t);
-    if (t == nA - 1) end_block(qA);
-    else if (t == T - 1) end_block(qB);
-  };
-
-#pragma unroll
-  for (int t = 0; t < D; ++t) issue(t);
-#pragma unroll
-  for (int i = 0; i < TQ; ++i)
-#pragma unroll
-    for (int dt = 0; dt < DT16; ++dt) o[i][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // ---- stage t: its copies are the only ones in flight; once every wave's have landed (and every wave has
+  // left stage t - 1, whose buffer is then free) stage t + 1 is requested ----
+  issue(0);
   begin_block(qA);
-  int t0 = 0;
 #pragma nounroll
-  for (; t0 + D <= T; t0 += D)
-    static_for<0, D>([&](auto uc) __attribute__((always_inline)) { iter(t0 + decltype(uc)::value, std::true_type{}); });
-  static_for<0, D - 1>([&](auto uc) __attribute__((always_inline)) {
-    if (t0 + decltype(uc)::value < T) iter(t0 + decltype(uc)::value, std::false_type{});
-  });
-  wait_vmcnt<0>();  // no copy may still be writing LDS when the workgroup ends
+  for (int t = 0; t < T; ++t) {
+    wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + 1 < T) issue(t + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(t);
+    if (t == nA - 1) {
+      end_block(qA, t);
+      if (t + 1 < T) begin_block(qB);
+    } else if (t == T - 1) {
+      end_block(qB, t);
+    }
+  }
 }
 
 // attn_seq_kernel: the attention of a batched call (nseq sequences of `rows` rows each, no mask) without

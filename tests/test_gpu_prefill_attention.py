@@ -1,0 +1,58 @@
+"""attn_prefill_kernel in its forms (query blocks alone or paired, four or twelve query tiles per workgroup)
+against attention in float64 and against the kernel that takes an explicit bias."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import log
+
+from test_gpu_seq_one import HEADS12, TINY, ULP2, _attention64, _vm
+
+from fast_dllm_relax_amd.params import TORCH_DTYPES
+from fast_dllm_relax_amd.runtime import build_prefix_block_attention_bias
+
+pytestmark = pytest.mark.gpu
+
+HEADS14 = dict(HEADS12, num_attention_heads=14, hidden_size=1792)  # 14 tiles: the last workgroup has two idle slots
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("kw,form", [(HEADS12, 0), (HEADS12, 2), (HEADS12, 3), (TINY, 1), (HEADS14, 1)],
+                         ids=["12 alone", "12 paired whole", "12 paired", "4", "14"])
+def test_prefill_attention_unmasked(monkeypatch, kw, form, dtype):
+    """Rows at the edges of query blocks (odd and even counts), keys at the edges of stages and key parts; a
+    growing last key makes the softmax renew its reference in the last block."""
+    vm = _vm(kw, dtype, monkeypatch, {"FDLLM_SEQ_ATTN": "0", "FDLLM_PREFILL_PAIR": str(form)})
+    td, nq, nkv, L = TORCH_DTYPES[dtype], kw["num_attention_heads"], kw["num_key_value_heads"], kw["num_hidden_layers"]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(11)
+    for rows, prefix in [(128, 0), (129, 0), (160, 31), (255, 1), (300, 84), (1056, 33)]:
+        cap = prefix + rows
+        rnd = lambda *s: torch.randn(s, device="cuda", generator=g).to(td)  # noqa: E731
+        q, k, v = rnd(1, rows, nq, 128), rnd(1, rows, nkv, 128), rnd(1, rows, nkv, 128)
+        k[:, -1] *= 6
+        kc, vc = rnd(L, 1, cap, nkv, 128), rnd(L, 1, cap, nkv, 128)
+        log(f"case: {rows} rows at {prefix}, {nq} / {nkv} heads, form {form}, {dtype}")
+        _, _, out = vm.attn_inplace(q, k, v, kc, vc, 0, prefix, 0, rows)
+        want = _attention64(q[0], kc[0, 0], vc[0, 0])
+        d = (out[0].double() - want).abs()
+        assert float(d.norm() / want.norm()) < ULP2[dtype], (rows, prefix, float(d.norm() / want.norm()))
+        assert float(d.max() / want.abs().max()) < 2 * ULP2[dtype], (rows, prefix)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_prefill_attention_block_causal(dtype):
+    """The block-causal rule as a key bound against the same rule as an explicit bias (attn_kernel)."""
+    vm = _vm(TINY, dtype)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(12)
+    for rows in (128, 129, 192, 353, 1025):
+        x = vm.embed(torch.randint(0, 999, (rows,), dtype=torch.int32, device="cuda", generator=g))[None]
+        blk = (rows - 1) // 32 * 32
+        bias = torch.from_numpy(build_prefix_block_attention_bias(blk, rows - blk, block_size=32)).cuda()
+        log(f"case: block-causal {rows} rows, {dtype}")
+        a, b = vm.forward_hidden(x, None).double(), vm.forward_hidden(x, bias).double()
+        # two layers of rounded tensors: each rounding (about 10 per layer) may flip by an ulp
+        assert float((a - b).norm() / b.norm()) < 4 * ULP2[dtype], rows
