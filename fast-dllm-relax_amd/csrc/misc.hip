@@ -105,17 +105,16 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const u16* h, int rows, 
 
 // The k-split sum + residual epilogue of an EPI_RESID projection (o_proj / down in a batched or
 // prefill-sized call) fused with the next RMSNorm.  The split sums come row-major (part[split][rows][hidden],
-// a part_rows GEMM launch).  A workgroup owns RPW rows.  Each 4-column unit adds its splits in split order
+// a part_rows GEMM launch).  A workgroup of NT threads owns RPW rows.  Each 4-column unit adds its splits in split order
 // (the requests of up to eight splits issued together), forms h = rnd(h + rnd(sum)) and the unit's sum of
 // squares as the split-sum kernel's epilogue does; a 16-column tile's sum is (g0 + g1) + (g2 + g3) of its
 // four units, again as there; h and the tile sums are written, and the rows are normalised exactly as
 // norm_rows_kernel does, from the same sums (kept in LDS with the new rows), into y (row-major, or with
 // yblk the large-M GEMMs' fragment blocks).
-template <int DT>
-__global__ __launch_bounds__(256) void resid_norm_kernel(const float* part, int splits, int rows, int hidden, u16* h,
-                                                         float* ssq, int ssq_ld, const u16* w, float eps, u16* y,
-                                                         int yblk) {
-  constexpr int RPW = 2;                // rows per workgroup
+template <int DT, int RPW, int NT>
+__global__ __launch_bounds__(NT) void resid_norm_kernel(const float* part, int splits, int rows, int hidden, u16* h,
+                                                        float* ssq, int ssq_ld, const u16* w, float eps, u16* y,
+                                                        int yblk) {
   constexpr int MAXH = 2048;            // hidden sizes up to this (the launcher checks)
   constexpr int SB = 8;                 // split sums requested at once
   __shared__ float gss[RPW][MAXH / 4];
@@ -124,7 +123,7 @@ __global__ __launch_bounds__(256) void resid_norm_kernel(const float* part, int 
   __shared__ float inv_s[RPW];
   const int r0 = blockIdx.x * RPW;
   const int nunits = hidden / 4, ntiles = hidden / 16;
-  for (int u = threadIdx.x; u < RPW * nunits; u += 256) {
+  for (int u = threadIdx.x; u < RPW * nunits; u += NT) {
     const int rl = u / nunits, n = 4 * (u - rl * nunits), m = r0 + rl;
     if (m >= rows) continue;
     f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -155,7 +154,7 @@ __global__ __launch_bounds__(256) void resid_norm_kernel(const float* part, int 
     gss[rl][n / 4] = ss;
   }
   __syncthreads();
-  for (int u = threadIdx.x; u < RPW * ntiles; u += 256) {
+  for (int u = threadIdx.x; u < RPW * ntiles; u += NT) {
     const int rl = u / ntiles, t = u - rl * ntiles, m = r0 + rl;
     if (m >= rows) continue;
     const float ts = (gss[rl][4 * t] + gss[rl][4 * t + 1]) + (gss[rl][4 * t + 2] + gss[rl][4 * t + 3]);
@@ -176,7 +175,7 @@ __global__ __launch_bounds__(256) void resid_norm_kernel(const float* part, int 
   }
   __syncthreads();
   const int ks = hidden / 32;
-  for (int u = threadIdx.x; u < RPW * (hidden / 8); u += 256) {
+  for (int u = threadIdx.x; u < RPW * (hidden / 8); u += NT) {
     const int rl = u % RPW, c = 8 * (u / RPW);
     const int r = r0 + rl;
     if (r >= rows) continue;
@@ -265,17 +264,25 @@ hipError_t launch_norm_rows(int dt, const uint16_t* h, int rows, int hidden, con
   return hipGetLastError();
 }
 
+template <int DT>
+static hipError_t launch_resid_norm_dt(const float* part, int splits, int rows, int hidden, uint16_t* h, float* ssq,
+                                       int ssq_ld, const uint16_t* w, float eps, uint16_t* y, int yblk, hipStream_t st) {
+  // a row per workgroup while its latency, not its traffic, is the launch (us, 1 / 2 rows per workgroup: 5.0 /
+  // 7.0 at 128 rows, even at 512, 17.6 / 11.4 at 2048)
+  if (rows <= 256)
+    hipLaunchKernelGGL((resid_norm_kernel<DT, 1, 384>), dim3(rows), dim3(384), 0, st, part, splits, rows, hidden, h, ssq,
+                       ssq_ld, w, eps, y, yblk);
+  else
+    hipLaunchKernelGGL((resid_norm_kernel<DT, 2, 256>), dim3((rows + 1) / 2), dim3(256), 0, st, part, splits, rows, hidden,
+                       h, ssq, ssq_ld, w, eps, y, yblk);
+  return hipGetLastError();
+}
+
 hipError_t launch_resid_norm(int dt, const float* part, int splits, int rows, int hidden, uint16_t* h, float* ssq,
                              int ssq_ld, const uint16_t* w, float eps, uint16_t* y, int yblk, hipStream_t st) {
   if (hidden % 32 || hidden > 2048 || splits < 1) return hipErrorInvalidValue;
-  const int wgs = (rows + 1) / 2;
-  if (dt == DT_BF16)
-    hipLaunchKernelGGL(resid_norm_kernel<DT_BF16>, dim3(wgs), dim3(256), 0, st, part, splits, rows, hidden, h, ssq, ssq_ld,
-                       w, eps, y, yblk);
-  else
-    hipLaunchKernelGGL(resid_norm_kernel<DT_F16>, dim3(wgs), dim3(256), 0, st, part, splits, rows, hidden, h, ssq, ssq_ld,
-                       w, eps, y, yblk);
-  return hipGetLastError();
+  if (dt == DT_BF16) return launch_resid_norm_dt<DT_BF16>(part, splits, rows, hidden, h, ssq, ssq_ld, w, eps, y, yblk, st);
+  return launch_resid_norm_dt<DT_F16>(part, splits, rows, hidden, h, ssq, ssq_ld, w, eps, y, yblk, st);
 }
 
 }  // namespace fdllm
