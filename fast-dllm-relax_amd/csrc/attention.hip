@@ -303,6 +303,13 @@ static hipError_t launch_dt(const AttnP& a, hipStream_t st) {
   return launch_loop<DT, 4, 2>(a, p, st);
 }
 
+hipError_t launch_rope_kv(int dt, const AttnP& a, hipStream_t st) {
+  if (a.nseq > 1 || a.rope == nullptr) return hipErrorInvalidValue;
+  if (dt == DT_BF16) hipLaunchKernelGGL(rope_kv_kernel<DT_BF16>, dim3(a.rows), dim3(128), 0, st, a);
+  else hipLaunchKernelGGL(rope_kv_kernel<DT_F16>, dim3(a.rows), dim3(128), 0, st, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_attention(int dt, const AttnP& a, hipStream_t st) {
   if (dt == DT_BF16) return launch_dt<DT_BF16>(a, st);
   return launch_dt<DT_F16>(a, st);

@@ -436,7 +436,7 @@ bool frag_chain(const fdllm_ctx* c, int rows) {
 //   per layer: qkv (RMSNorm on load, + bias) -> attention (RoPE, KV append, GQA) -> o_proj + residual
 //              -> gate_up (RMSNorm on load, SiLU * up) -> down + residual
 // kv: per-layer cache base pointers are k/v + layer * layer_stride (elements).  out == nullptr skips
-// the final norm (build_prefix_cache returns only the caches).
+// the final norm (build_prefix_cache returns only the caches), and all of the last layer past its K/V rows.
 // sb: a batched call (rows = sb->nseq x sb->rows; pos_dev holds one offset per sequence).
 int run_layers(fdllm_ctx* c, const void* x_in, int rows, uint16_t* kbase, uint16_t* vbase, size_t layer_stride,
                int write_start, const int32_t* pos_dev, int attend_len, int mask, const float* bias,
@@ -484,6 +484,11 @@ int run_layers(fdllm_ctx* c, const void* x_in, int rows, uint16_t* kbase, uint16
     }
     rc = run_gemm(c, CFG_QKV, g.q, 1, st);
     if (rc) return rc;
+    if (out == nullptr && l + 1 == f.num_hidden_layers) {
+      // build_prefix_cache returns the caches only, and the last layer's end with its K/V rows
+      if (!at.roped) HIPCHK(launch_rope_kv(f.dtype, at, st));
+      break;
+    }
     HIPCHK(launch_attention(f.dtype, at, st));
     // o_proj + the post-attention norm: with a forced k split, when gate_up takes normalised rows
     bool gu_ready = false;

@@ -260,6 +260,8 @@ bool attn_takes_roped(const AttnP& a);
 // the splits need (0 without splits).
 size_t plan_seq_units(AttnP& a, int ncu);
 hipError_t launch_attention(int dt, const AttnP& a, hipStream_t st);
+// only the RoPE and the append of the call's K/V rows (rope_kv_kernel; one sequence)
+hipError_t launch_rope_kv(int dt, const AttnP& a, hipStream_t st);
 size_t attn_partial_floats(const AttnP& a);
 
 

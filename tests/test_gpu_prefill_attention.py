@@ -56,3 +56,30 @@ def test_prefill_attention_block_causal(dtype):
         a, b = vm.forward_hidden(x, None).double(), vm.forward_hidden(x, bias).double()
         # two layers of rounded tensors: each rounding (about 10 per layer) may flip by an ulp
         assert float((a - b).norm() / b.norm()) < 4 * ULP2[dtype], rows
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_prefill_stops_at_the_last_layers_cache_rows(dtype):
+    """build_prefix_cache leaves out what follows the last layer's K/V rows: the caches of a two-layer model
+    are the first two layers' of a three-layer one, bit for bit, on every attention kernel's row counts, with
+    and without a bias."""
+    from fast_dllm_relax_amd.config import FastDLLMConfig
+    from fast_dllm_relax_amd.params import random_params_torch
+    from fast_dllm_relax_amd.vm import HipVM
+
+    c3, c2 = FastDLLMConfig(**dict(TINY, num_hidden_layers=3)), FastDLLMConfig(**TINY)
+    params = random_params_torch(c3, 5, dtype=dtype)
+    vm3, vm2 = HipVM(c3, params, dtype=dtype), HipVM(c2, params[:1 + 14] + params[1 + 21:], dtype=dtype)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(13)
+    for rows in (1, 20, 32, 33, 100, 128, 300):
+        x = vm3.embed(torch.randint(0, 999, (rows,), dtype=torch.int32, device="cuda", generator=g))[None]
+        full = torch.zeros((1, 1, rows, rows), device="cuda")
+        for bias in (None, full):
+            log(f"case: build_prefix_cache {rows} rows, bias {bias is not None}, {dtype}")
+            caches = []
+            for vm, L in ((vm3, 3), (vm2, 2)):
+                k = torch.zeros((L, 1, rows + 3, 2, 128), dtype=TORCH_DTYPES[dtype], device="cuda")
+                caches.append(vm.build_prefix_cache(x, bias, k, torch.zeros_like(k)))
+            for a, b in zip(*caches):
+                assert torch.equal(a[:2].view(torch.int16), b.view(torch.int16)), (rows, bias is None)
