@@ -205,7 +205,18 @@ static_assert(WrTiny::lds >= (size_t)4 * 1 * 4 * 64 * 8 && WrSmall::lds >= (size
 // 64 row blocks of 8192 rows fill 512 slots, two per compute unit, where the 128 x 256 blocks' 384
 // leave half the units with one)
 using WrB3 = WrCfg<8, 3, FD_WR_DEPTH>;
-enum MmId : int { MM_SMALL = 0, MM_WIDE = 1, MM_WIDE_D = 2, MM_BIG = 3, MM_WT = 4, MM_WR = 5, MM_WR_S = 6, MM_WR_M = 7, MM_WR_T = 8, MM_WR_3 = 9, MM_WT_8 = 10, MM_WT_256 = 11 };
+// k-grouped register-weight kernel (gemm_wt.hpp, gemm_wk_kernel): NWN x KP waves of 16 MF rows x TPW tiles
+template <int MF, int TPW, int NWN, int KP, int D>
+struct WkCfg {
+  static constexpr int mf = MF, tpw = TPW, nwn = NWN, kp = KP, d = D;
+  static constexpr int bm = 16 * MF, bn_tiles = NWN * TPW, kss = KP;
+  static constexpr size_t lds_in = (size_t)(D + 1) * KP * MF * 1024, lds_red = (size_t)KP * NWN * TPW * MF * 1024;
+  static constexpr size_t lds = lds_in > lds_red ? lds_in : lds_red;
+};
+using WkGu4 = WkCfg<4, 2, 3, 2, 4>;  // (depth 3 to 12 and one k group measure the same, four k groups 1.5 us more)
+using WkGu6 = WkCfg<6, 2, 3, 2, 4>;
+using WkGu8 = WkCfg<8, 2, 3, 2, 3>;
+enum MmId : int { MM_SMALL = 0, MM_WIDE = 1, MM_WIDE_D = 2, MM_BIG = 3, MM_WT = 4, MM_WR = 5, MM_WR_S = 6, MM_WR_M = 7, MM_WR_T = 8, MM_WR_3 = 9, MM_WT_8 = 10, MM_WT_256 = 11, MM_WK_GU4 = 12, MM_WK_GU6 = 13, MM_WK_GU8 = 14 };
 struct MmInfo { int bm, bn_tiles, kss; };
 template <class M> constexpr MmInfo mm_info_of() { return MmInfo{M::bm, M::bn_tiles, M::kss}; }
 static MmInfo mm_info(int id) {
@@ -221,6 +232,9 @@ static MmInfo mm_info(int id) {
     case MM_WR_3: return mm_info_of<WrB3>();
     case MM_WT_8: return mm_info_of<WtBig8>();
     case MM_WT_256: return mm_info_of<WtB256>();
+    case MM_WK_GU4: return mm_info_of<WkGu4>();
+    case MM_WK_GU6: return mm_info_of<WkGu6>();
+    case MM_WK_GU8: return mm_info_of<WkGu8>();
     default: return mm_info_of<MmSmall>();
   }
 }
@@ -244,15 +258,27 @@ static int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
   // 512 (but 19.4 / 21.2 at 1024); o_proj 12.8 / 11.9, 12.8 / 11.9, 14.0 / 12.0 (15.1 / 21.4 at 1024)
   if (M >= 33 && ((pol.wr_small_ops >> cfg) & 1) && (cfg == CFG_QKV || (cfg == CFG_OPROJ && M < 2048)))
     return M <= 512 ? MM_WR_T : MM_WR_S;
-  // gate_up and down below 256 rows: register-weight blocks too (us per launch, gate_up including its norm
-  // pass; LDS-staged kernel / 64 x 128 / 128 x 128 blocks): gate_up 24.8 / 21.3 / 22.7 at 64 rows, 30.0 /
-  // 29.9 / 26.1 at 128, 38.6 / 29.5 / 35.6 at 192; down 21.4 / 16.8 / 18.0, 21.4 / 18.0 / 20.8, 27.1 / 24.7 /
-  // 25.2.  The 128 x 128 blocks win where they make one round of workgroups and the 64 x 128 ones two.
-  if (M >= 33 && M < 256 && (cfg == CFG_GATE_UP || cfg == CFG_DOWN)) {
+  // gate_up and down of short calls: register-weight blocks too (FDLLM_WR_FFN picks 64 x 128 or 128 x 128 blocks
+  // below 1024 rows, or the LDS-staged kernels).
+  if (M >= 33 && M < 1024 && pol.wr_ffn >= 0 && (cfg == CFG_GATE_UP || cfg == CFG_DOWN)) {
     const int sh = cfg == CFG_GATE_UP ? 0 : 1;
-    const int ffn = pol.wr_ffn >= 0 ? pol.wr_ffn : (M > 64 && M <= 128 ? 4 | 2 : 1 | 2);
-    if ((ffn >> sh) & 1) return MM_WR_S;
-    if ((ffn >> (sh + 2)) & 1) return MM_WR_M;
+    if ((pol.wr_ffn >> sh) & 1) return MM_WR_S;
+    if ((pol.wr_ffn >> (sh + 2)) & 1) return MM_WR_M;
+  } else if (M >= 33 && cfg == CFG_GATE_UP) {
+    // us per launch including its norm pass, k groups / 64 x 128 / 128 x 128 / LDS-staged blocks: 33 rows 17.5 /
+    // 20.5, 64 rows 18.5 / 21.0 / 22.7, 96 rows 20.5 / - / 24.1, 128 rows 23.3 / 29.9 / 26.0, 129 rows 30.8 / 27.2 /
+    // 31.6, 192 rows 32.5 / 28.8 / 34.2, 208 rows - / 34.5 / 35.0, 256 rows 37.6 / 37.5 / 37.1 / 43.2, 320 rows - / 37.8
+    // / 34.9 / 41.7, 384 rows - / 43.2 / 36.6 / 42.1, 416 rows - / 44.3 / 43.0 / 42.0, 512 rows - / 54.1 / 48.8 / 42.6
+    if (M <= 128 && ntiles % WkGu8::bn_tiles == 0) return M <= 64 ? MM_WK_GU4 : M <= 96 ? MM_WK_GU6 : MM_WK_GU8;
+    if (M <= 224) return MM_WR_S;
+    if (M <= 400) return MM_WR_M;
+  } else if (M >= 33 && cfg == CFG_DOWN) {
+    // us per launch with its split sum, 64 x 128 blocks / LDS-staged: 64 rows 14.4 / 21.4, 128 rows 15.7 / 21.4, 192
+    // rows 16.7 / 27.1, 256 rows 17.8 / 22.6, 320 rows 20.9 / 23.8, 352 rows 27.7 / 24.1.  From 417 to 672 rows
+    // 128 x 128 blocks: in a prefill, us per layer against the LDS-staged blocks: 448 rows 90.7 / 93.0, 509 rows
+    // 91.6 / 93.5, 576 rows 102.4 / 109.3, 640 rows 104.9 / 111.3 (but 384 rows 95.4 / 88.5, 768 rows 126.3 / 120.6)
+    if (M <= 320) return MM_WR_S;
+    if (M > 416 && M <= 672) return MM_WR_M;
   }
   switch (cfg) {
     case CFG_LM_HEAD: return MM_WIDE;  // one 256-column confidence tile per block column
@@ -296,7 +322,7 @@ GemmPlan gemm_plan(int cfg, GemmP& a, int stream_split, const MmPolicy& pol) {
       // measured 3.92 against 3.94-3.95 ms per batched step (fewer partials for the split sum; five
       // splits 4.03, ten 3.95)
       if (cfg == CFG_DOWN && a.M > 128) target = target * 7 / 8;
-      if (id == MM_WT_256) target = 0;  // no split
+      if (id == MM_WT_256 || (id >= MM_WK_GU4 && id <= MM_WK_GU8)) target = 0;  // no split
       int split = 1;
       const int max_split = id == MM_WR || id == MM_WR_S || id == MM_WR_M || id == MM_WR_T || id == MM_WR_3 ? 16 : 8;
       if (pol.force_split > 1 && cfg != CFG_LM_HEAD && nst % pol.force_split == 0 && nst / pol.force_split >= pol.min_stages)
@@ -304,6 +330,15 @@ GemmPlan gemm_plan(int cfg, GemmP& a, int stream_split, const MmPolicy& pol) {
       else
         for (int d = 2; d <= max_split && wgs * split < target && cfg != CFG_LM_HEAD; ++d)
           if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
+      if (cfg == CFG_DOWN && id == MM_WR_S && pol.wr_ffn < 0 && pol.force_split <= 1 && pol.target_wgs >= 256) {
+        // down's 64 x 128 blocks: the most splits up to seven that leave every XCD a workgroup per compute unit
+        // at most (us per launch with its split sum; 130 rows: 5 splits 16.7, 7 splits 21.5, of 35 workgroups on
+        // seven XCDs; 64 rows: 7 splits 14.4, 14 splits 16.8, whose partials cost more than their workgroups give)
+        const int fit = std::min(7, std::max(1, pol.target_wgs / 8 / ((wgs + 7) / 8)));
+        split = 1;
+        for (int d = 2; d <= fit; ++d)
+          if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
+      }
       p.ksplit = split;
       a.kps = a.KS / split;
       p.part_floats = split > 1 ? (size_t)split * a.ntiles * ((a.M + 15) / 16) * 256 : 0;
@@ -445,6 +480,27 @@ static hipError_t launch_wt_cfg(const GemmP& a, const GemmPlan& p, hipStream_t s
   return hipGetLastError();
 }
 
+template <int DT, int EPI, class W>
+static hipError_t launch_wk_cfg(const GemmP& a, const GemmPlan& p, hipStream_t st) {
+  auto kern = gemm_wk_kernel<DT, EPI, W::mf, W::tpw, W::nwn, W::kp, W::d>;
+  if (a.KS % (p.ksplit * W::kp)) return hipErrorInvalidValue;
+  static bool attr = false;  // per instantiation
+  if (!attr) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)W::lds) !=
+        hipSuccess)
+      (void)hipGetLastError();
+    attr = true;
+  }
+  const int total = p.nbm * p.nbn, per = (total + 7) / 8;
+  hipLaunchKernelGGL(kern, dim3(8 * per, p.ksplit), dim3(64 * W::nwn * W::kp), W::lds, st, a, p.nbm, p.nbn);
+  if (p.ksplit > 1 && !a.part_rows) {
+    const int nblk = (a.M + 15) / 16;
+    hipLaunchKernelGGL((gemm_mm_split_epilogue_kernel<DT, EPI>), dim3((a.N + 15) / 16, (nblk + 3) / 4), dim3(256), 0,
+                       st, a, p.ksplit);
+  }
+  return hipGetLastError();
+}
+
 // GK_MM rows arrive normalised (see GemmKind), so every large-M launch runs without the norm transform.
 template <int DT, int CFG, class C>
 static hipError_t launch_mm(const GemmP& a, const GemmPlan& p, hipStream_t st) {
@@ -466,6 +522,9 @@ static hipError_t launch_mm(const GemmP& a, const GemmPlan& p, hipStream_t st) {
     return hipErrorInvalidValue;
   }
   if constexpr (CFG == CFG_GATE_UP) {
+    if (p.mm_id == MM_WK_GU4) return launch_wk_cfg<DT, C::epi, WkGu4>(a, p, st);
+    if (p.mm_id == MM_WK_GU6) return launch_wk_cfg<DT, C::epi, WkGu6>(a, p, st);
+    if (p.mm_id == MM_WK_GU8) return launch_wk_cfg<DT, C::epi, WkGu8>(a, p, st);
     if (p.mm_id == MM_WT_256) return launch_wt_cfg<DT, C::epi, WtB256>(a, p, st);
     if (p.mm_id == MM_WT) return launch_wt_cfg<DT, C::epi, WtBig>(a, p, st);
     if (p.mm_id == MM_WT_8) return launch_wt_cfg<DT, C::epi, WtBig8>(a, p, st);

@@ -474,4 +474,153 @@ void gemm_wr_kernel(GemmP a, int nbm, int nbn) {
   }
 }
 
+// Register weights as in gemm_wr_kernel, with the k steps dealt to KP groups of waves: wave (wn, kp) of NWN x KP
+// owns TPW weight tiles (a block is 16 MF rows x 16 NWN TPW columns) for k steps kp, kp + KP, ...; a stage is KP k
+// steps, whose activation blocks the NWN waves of each group copy and share in LDS.  The groups' sums are added
+// in LDS at the end, in group order, group kp finishing the row blocks f with f % KP == kp.
+//
+// For calls of 33 to 128 rows, whose launches are bound by what a compute unit takes in: (rows + columns) x 3 KB
+// per workgroup at hidden 1536.  Columns are chosen so that one round of workgroups covers the chip with as few
+// bytes each as possible, and the k groups put more waves, hence more loads in flight, on each compute unit
+// than the columns alone would (figures at mm_choice).
+template <int DT, int EPI, int MF, int TPW, int NWN, int KP, int D>
+__global__ __launch_bounds__(64 * NWN * KP) __attribute__((amdgpu_waves_per_eu((NWN * KP + 3) / 4, (NWN * KP + 3) / 4)))
+void gemm_wk_kernel(GemmP a, int nbm, int nbn) {
+  constexpr int R = D + 1;
+  constexpr int DPW = (MF + NWN - 1) / NWN;  // activation blocks each wave copies per stage (past the last: the last again)
+  constexpr int VPS = TPW + DPW;             // vector memory instructions per wave per stage
+  static_assert(D >= 2 && (D - 1) * VPS < 64, "outstanding copies fit the memory counter");
+  static_assert(EPI != EPI_SILU_PAIR || TPW % 2 == 0, "gate/up pairs stay within a wave");
+  static_assert(MF % KP == 0, "the groups finish as many row blocks each");
+  static_assert(EPI != EPI_LOGITS, "no confidence tiles here");
+  extern __shared__ __align__(16) unsigned char smem[];  // [R][KP][MF][1 KB]
+
+  const int total = nbm * nbn;
+  const int per = (total + 7) / 8;
+  const int logical = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);  // (XCD order, as gemm_wr_kernel)
+  if (logical >= total) return;
+  const int nb = logical / nbm, mb = logical - nb * nbm;
+
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wn = w % NWN, kp = w / NWN;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int m0 = mb * 16 * MF, mlast = a.M - 1;
+  const int tw0 = (nb * NWN + wn) * TPW, tlast = a.ntiles - 1;  // this wave's first tile
+  const int ks = a.KS / (int)gridDim.y, kb = (int)blockIdx.y * ks + kp;  // the split's k steps; this group's first
+  const int nst = ks / KP;  // (the plan takes whole stages)
+
+  const u16* xs[DPW];
+  size_t xstep[DPW];
+#pragma unroll
+  for (int q = 0; q < DPW; ++q) {
+    const int i = min(wn + NWN * q, MF - 1);
+    if (a.xfrag == 2) {
+      const int b = min(m0 / 16 + i, mlast / 16);
+      xs[q] = a.X + ((size_t)b * a.KS + kb) * 512 + 8 * lane;
+      xstep[q] = 512 * KP;
+    } else {
+      const int m = min(m0 + 16 * i + lr, mlast);
+      xs[q] = a.X + (size_t)m * a.ldx + 32 * kb + 8 * lg;
+      xstep[q] = 32 * KP;
+    }
+  }
+  const u16* ws[TPW];
+#pragma unroll
+  for (int j = 0; j < TPW; ++j) ws[j] = a.W + ((size_t)min(tw0 + j, tlast) * a.KS + kb) * 512 + 8 * lane;
+
+  u32x4 wv[R][TPW];
+  auto issue = [&](int st, u32x4 (&dst)[TPW], int buf) {
+    const int s = min(st, nst - 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < TPW; ++j) dst[j] = FD_WLOAD(reinterpret_cast<const u32x4*>(ws[j] + (size_t)s * (512 * KP)));
+#pragma unroll
+    for (int q = 0; q < DPW; ++q)
+      lds_copy16(xs[q] + (size_t)s * xstep[q], smem + (((size_t)buf * KP + kp) * MF + min(wn + NWN * q, MF - 1)) * 1024);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  f32x4 acc[TPW][MF];
+#pragma unroll
+  for (int j = 0; j < TPW; ++j)
+#pragma unroll
+    for (int f = 0; f < MF; ++f) acc[j][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < D; ++u) issue(u, wv[u], u);
+
+  // stages as in gemm_wr_kernel's piped form: the wait of stage st is for stage st + 1's copies and weights, and
+  // stage st + 1's fragments are read right after stage st's MFMAs
+  const u32x4* lds = reinterpret_cast<const u32x4*>(smem) + (size_t)kp * MF * 64;
+  u32x4 xf[MF];
+  wait_vmcnt<(D - 1) * VPS>();  // stage 0
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int f = 0; f < MF; ++f) xf[f] = lds[f * 64 + lane];
+  auto stage = [&](int st, auto uc, auto exact) {
+    constexpr int u = decltype(uc)::value;
+    if constexpr (decltype(exact)::value) wait_vmcnt<(D - 2) * VPS>();
+    else wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    issue(st + D, wv[(u + D) % R], (u + D) % R);
+#pragma unroll
+    for (int j = 0; j < TPW; ++j)
+#pragma unroll
+      for (int f = 0; f < MF; ++f) acc[j][f] = mfma16<DT>(wv[u][j], xf[f], acc[j][f]);
+    const u32x4* nblk = lds + (size_t)((u + 1) % R) * KP * MF * 64;
+#pragma unroll
+    for (int f = 0; f < MF; ++f) xf[f] = nblk[f * 64 + lane];
+  };
+  int st0 = 0;
+#pragma nounroll
+  for (; st0 + R <= nst; st0 += R)
+    static_for<0, R>([&](auto uc) { stage(st0 + decltype(uc)::value, uc, std::true_type{}); });
+  static_for<0, R - 1>([&](auto uc) {
+    if (st0 + decltype(uc)::value < nst) stage(st0 + decltype(uc)::value, uc, std::false_type{});
+  });
+  wait_vmcnt<0>();  // no copy may still be writing LDS when the sums go through it
+  __syncthreads();
+
+  // the groups' sums: every wave leaves the row blocks other groups finish, and adds the others' of its own
+  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [KP][NWN][TPW][MF][64]
+#pragma unroll
+  for (int j = 0; j < TPW; ++j)
+#pragma unroll
+    for (int f = 0; f < MF; ++f)
+      if (f % KP != kp) red[((((size_t)kp * NWN + wn) * TPW + j) * MF + f) * 64 + lane] = acc[j][f];
+  __syncthreads();
+  static_for<0, KP>([&](auto kc) {
+    constexpr int K0 = decltype(kc)::value;
+    if (kp != K0) return;
+#pragma unroll
+    for (int f = K0; f < MF; f += KP) {
+#pragma unroll
+      for (int j = 0; j < TPW; ++j) {
+        f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < KP; ++k) {
+          const f32x4 v = k == K0 ? acc[j][f] : red[((((size_t)k * NWN + wn) * TPW + j) * MF + f) * 64 + lane];
+          sum = k == 0 ? v : sum + v;
+        }
+        acc[j][f] = sum;
+      }
+      if (gridDim.y > 1) {
+#pragma unroll
+        for (int j = 0; j < TPW; ++j) store_split_unit(a, blockIdx.y, tw0 + j, mb * MF + f, lane, acc[j][f]);
+      } else if constexpr (EPI == EPI_SILU_PAIR) {
+#pragma unroll
+        for (int p = 0; p < TPW / 2; ++p) {
+          const f32x4 v[2] = {acc[2 * p][f], acc[2 * p + 1][f]};
+          os_epilogue<DT, EPI, 2, false>(a, v, m0 + 16 * f + lr, tw0 + 2 * p, lg);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < TPW; ++j) {
+          const f32x4 v[1] = {acc[j][f]};
+          os_epilogue<DT, EPI, 1, false>(a, v, m0 + 16 * f + lr, tw0 + j, lg);
+        }
+      }
+    }
+  });
+}
+
 }  // namespace fdllm

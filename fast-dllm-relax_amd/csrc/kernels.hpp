@@ -121,8 +121,8 @@ struct MmPolicy {
   int wr_ops = (1 << CFG_QKV) | (1 << CFG_OPROJ) | (1 << CFG_GATE_UP) | (1 << CFG_DOWN) | (1 << CFG_LM_HEAD);
   int wr_min_rows = 0;
   int wr_small_ops = (1 << CFG_QKV) | (1 << CFG_OPROJ);  // take the 64 x 128 register-weight blocks below the 128 x 256 ones
-  // gate_up / down below 256 rows: -1 the measured choice of register-weight blocks, else bit 0 / 1 the 64 x 128
-  // blocks, bit 2 / 3 the 128 x 128 ones (0: the LDS-staged kernel)
+  // gate_up / down below 1024 rows: -1 the measured choice, else bit 0 / 1 the 64 x 128 register-weight blocks,
+  // bit 2 / 3 the 128 x 128 ones (0: the LDS-staged kernels)
   int wr_ffn = -1;
   int force_split = 0;  // > 1: this k split whenever it divides the stages (the fused o_proj + norm)
   int wr3 = 1;          // o_proj / down at the register-weight thresholds: 128 x 192 blocks (0: 128 x 256)
