@@ -247,6 +247,21 @@ static int wr_default_min_rows(int cfg) {
   return cfg == CFG_GATE_UP || cfg == CFG_DOWN ? 2048 : 4096;
 }
 static int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
+  // The large blocks by how their counts fill the 256 compute units (two workgroups each), us per launch.
+  // Register-weight 128 x 256 gate_up of 641 to 896 rows, one round of at most 490 blocks / LDS-staged: 50.7 /
+  // 56.7 at 660 rows, 51.7 / 59.4 at 896 (but 51.3 / 43.9 at 640, 68.3 / 59.1 at 900).  o_proj past 2560 rows, where
+  // its 64 x 128 blocks start a second round: register-weight 128 x 192 / 64 x 128: 28.6 / 36.0 at 2700, 28.8 / 36.7
+  // at 3000 (28.5 / 23.9 at 2560).  Down, register-weight 128 x 192 / LDS-staged: 31.9 / 33.8 at 680 rows, 37.6 / 40.3
+  // at 896, 39.4 / 41.3 at 1024, 55.5 / 52.5 at 1100, 59.9 / 59.4 at 1400, 61.7 / 64.1 at 1600, 101 / 97 at 2800, 98 / 105
+  // at 3500; 128 x 256 where their splits come to one round, 47.8 / 53.4 at 1200, 78.6 / 86.9 at 2100, 79.4 / 90.1 at 2400.
+  if (pol.wr_min_rows == 0 && ((pol.wr_ops >> cfg) & 1) && pol.wr_ffn < 0) {
+    const bool b3 = pol.wr3 && ntiles % WrB3::bn_tiles == 0;
+    if (cfg == CFG_GATE_UP && M > 640 && M <= 896) return MM_WR;
+    if (cfg == CFG_OPROJ && M > 2560 && b3) return MM_WR_3;
+    if (cfg == CFG_DOWN && ((M > 1024 && M <= 1280) || (M > 2048 && M <= 2560))) return MM_WR;
+    if (cfg == CFG_DOWN && ((M > 672 && M <= 1024) || (M > 1536 && M <= 2048)) && b3) return MM_WR_3;
+    if (cfg == CFG_DOWN && M > 2560 && M <= 3200 && ntiles % WtBig::bn_tiles == 0) return MM_WT;
+  }
   const int min_rows = pol.wr_min_rows > 0 ? pol.wr_min_rows : wr_default_min_rows(cfg);
   if (M >= std::max(min_rows, 33) && ((pol.wr_ops >> cfg) & 1))
     return pol.wr3 && (cfg == CFG_OPROJ || cfg == CFG_DOWN) && ntiles % WrB3::bn_tiles == 0 ? MM_WR_3 : MM_WR;
@@ -256,7 +271,8 @@ static int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
   // 23.3 / 26.4 at 2048 (equal below 384).  Up to 512 rows 64 x 64 blocks, twice the workgroups, do better
   // still (us, 64 x 128 / 64 x 64 blocks): qkv 14.4 / 13.4 at 128 rows, 15.7 / 13.7 at 256, 16.8 / 14.9 at
   // 512 (but 19.4 / 21.2 at 1024); o_proj 12.8 / 11.9, 12.8 / 11.9, 14.0 / 12.0 (15.1 / 21.4 at 1024)
-  if (M >= 33 && ((pol.wr_small_ops >> cfg) & 1) && (cfg == CFG_QKV || (cfg == CFG_OPROJ && M < 2048)))
+  // o_proj up to 1344 rows, one round of 64 x 128 blocks (16.1 / 20.0 at 1300 rows, 25.9 / 23.3 at 1500)
+  if (M >= 33 && ((pol.wr_small_ops >> cfg) & 1) && (cfg == CFG_QKV || (cfg == CFG_OPROJ && M <= 1344)))
     return M <= 512 ? MM_WR_T : MM_WR_S;
   // gate_up and down of short calls: register-weight blocks too (FDLLM_WR_FFN picks 64 x 128 or 128 x 128 blocks
   // below 1024 rows, or the LDS-staged kernels).
@@ -330,6 +346,12 @@ GemmPlan gemm_plan(int cfg, GemmP& a, int stream_split, const MmPolicy& pol) {
       else
         for (int d = 2; d <= max_split && wgs * split < target && cfg != CFG_LM_HEAD; ++d)
           if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
+      if (cfg == CFG_DOWN && id == MM_WR && pol.wr_min_rows == 0 && pol.force_split <= 1 && pol.target_wgs >= 256) {
+        // (one round: at 1152 rows five splits of 54 blocks took 58.9 us, at 1200 four of 60 blocks 47.8)
+        split = 1;
+        for (int d = 2; d <= max_split && wgs * d <= pol.target_wgs; ++d)
+          if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
+      }
       if (cfg == CFG_DOWN && id == MM_WR_S && pol.wr_ffn < 0 && pol.force_split <= 1 && pol.target_wgs >= 256) {
         // down's 64 x 128 blocks: the most splits up to seven that leave every XCD a workgroup per compute unit
         // at most (us per launch with its split sum; 130 rows: 5 splits 16.7, 7 splits 21.5, of 35 workgroups on

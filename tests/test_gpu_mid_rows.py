@@ -1,4 +1,4 @@
-"""The projections' kernels of 33 to 672 rows: the k-grouped register-weight gate_up (33 to 128 rows) and the
+"""The projections' kernels of 33 to 3201 rows: the k-grouped register-weight gate_up (33 to 128 rows) and the
 block and split choices around it, at the edges of each one's rows."""
 
 from __future__ import annotations
@@ -26,7 +26,8 @@ def test_mid_rows_match_the_lds_staged_kernels(monkeypatch, kw, dtype):
                                        "FDLLM_FUSE_OPROJ": "0", "FDLLM_FUSE_DOWN": "0"})
     g = torch.Generator(device="cuda")
     g.manual_seed(17)
-    for rows in (33, 48, 63, 64, 65, 96, 97, 127, 128, 129, 224, 225, 320, 321, 400, 401, 417, 672, 673):
+    for rows in (33, 48, 63, 64, 65, 96, 97, 127, 128, 129, 224, 225, 320, 321, 400, 401, 417, 640, 641, 672, 673, 896, 897,
+                 1024, 1025, 1280, 1281, 1344, 1345, 1537, 2049, 2560, 2561, 3201):
         x = vm.embed(torch.randint(0, 999, (rows,), dtype=torch.int32, device="cuda", generator=g))[None]
         log(f"case: forward_hidden {rows} rows, {kw['hidden_size']} x {kw['intermediate_size']}, {dtype}")
         a, b = vm.forward_hidden(x, None).double(), ref.forward_hidden(x, None).double()
