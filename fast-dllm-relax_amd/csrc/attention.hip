@@ -140,7 +140,7 @@ static hipError_t launch_loop(const AttnP& a, const AttnPlan& p, hipStream_t st)
   return hipGetLastError();
 }
 
-template <int DT, int CH, int KH, int MASK, int QPW>
+template <int DT, int CH, int KH, int MASK, int QPW, bool WIN = false>
 static hipError_t launch_chunk_kh(const AttnP& a, const AttnPlan& p, hipStream_t st) {
   // K and V^T of the chunk, then (one-sequence calls) the queries the first key part shares
   const size_t loop_lds = (size_t)CH * KLD * 2 + (size_t)HD * (CH + 8) * 2 +
@@ -149,7 +149,7 @@ static hipError_t launch_chunk_kh(const AttnP& a, const AttnPlan& p, hipStream_t
   const size_t lds = std::max(loop_lds, merge_lds);
   if (lds > 160 * 1024) return hipErrorInvalidValue;
   const int nseq = std::max(a.nseq, 1);
-  auto kern = attn_chunk_kernel<DT, QPW, KH, CH, MASK>;
+  auto kern = attn_chunk_kernel<DT, QPW, KH, CH, MASK, WIN>;
   raise_lds(kern, lds);
   if (nseq == 1)
     hipLaunchKernelGGL(kern, dim3(attn_chunk_grid_1seq(p.qg, a.nkv, a.S)), dim3(64 * QPW * KH), lds, st, a);
@@ -166,6 +166,12 @@ static hipError_t launch_chunk_kh(const AttnP& a, const AttnPlan& p, hipStream_t
 template <int DT, int CH, int MASK>
 static hipError_t launch_chunk_shape(const AttnP& a, const AttnPlan& p, hipStream_t st) {
   if (p.key_groups != 2) return hipErrorInvalidValue;
+  if (a.kwin != nullptr) {
+    if constexpr (MASK == 0) {
+      if (p.q_tiles_per_wg == 2 && a.rope == nullptr) return launch_chunk_kh<DT, CH, 2, 0, 2, true>(a, p, st);
+    }
+    return hipErrorInvalidValue;
+  }
   if (p.q_tiles_per_wg == 2) return launch_chunk_kh<DT, CH, 2, MASK, 2>(a, p, st);
   if (p.q_tiles_per_wg == 4) return launch_chunk_kh<DT, CH, 2, MASK, 4>(a, p, st);
   return hipErrorInvalidValue;
@@ -285,7 +291,7 @@ static hipError_t launch_dt(const AttnP& a, hipStream_t st) {
     return launch_seq<DT>(a, st);
   }
   const AttnPlan p = attn_plan(a.rows, a.nq, a.nkv, a.Lk, a.target_wgs, a.nseq, a.mask, a.ncu);
-  if (p.seq || (a.roped && !attn_takes_roped(a))) return hipErrorInvalidValue;
+  if (p.seq || (a.roped && !attn_takes_roped(a)) || (a.kwin != nullptr && !p.chunked)) return hipErrorInvalidValue;
   if (p.S != a.S || p.chunk != a.chunk) return hipErrorInvalidValue;
   if (a.ofrag && (a.nseq > 1 || a.rows > 32)) return hipErrorInvalidValue;
   if (a.nseq > MAX_SEQS) return hipErrorInvalidValue;
@@ -301,6 +307,11 @@ static hipError_t launch_dt(const AttnP& a, hipStream_t st) {
   }
   if (p.key_groups == 1) return launch_loop<DT, 4, 1>(a, p, st);
   return launch_loop<DT, 4, 2>(a, p, st);
+}
+
+bool attn_takes_window(const AttnP& a) {
+  return a.nseq <= 1 && !a.seq_attn &&
+         attn_plan(a.rows, a.nq, a.nkv, a.Lk, a.target_wgs, a.nseq, a.mask, a.ncu).chunked;
 }
 
 hipError_t launch_rope_kv(int dt, const AttnP& a, hipStream_t st) {

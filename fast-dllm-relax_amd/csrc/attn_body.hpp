@@ -357,7 +357,7 @@ __device__ __forceinline__ void attn_chunk_qload(const AttnP& a, int bx, int by,
 // consecutive lanes take 16 key quads x 2 dim chunks of V, so the LDS stores of attn_chunk_compute hit 64 distinct banks
 // per pass (rows are 68 dwords apart, 4 banks on).  Rows past kend read row kbeg and are masked or
 // zeroed later.
-template <int QPW, int KH, int CH, bool WCS = false>
+template <int QPW, int KH, int CH, bool WCS = false, bool WIN = false>
 __device__ __forceinline__ void attn_chunk_load(const AttnP& a, int by, int bz, AttnChunkRegs<QPW, KH, CH, WCS>& R,
                                                 int tid) {
   typedef AttnChunkRegs<QPW, KH, CH, WCS> Regs;
@@ -366,8 +366,10 @@ __device__ __forceinline__ void attn_chunk_load(const AttnP& a, int by, int bz, 
   const size_t krow = (size_t)a.nkv * HD;
   const int kbeg = bz * a.chunk;
   const int kend = min(kbeg + a.chunk, a.Lk);
-  const u16* kq_base = a.qkv + a.nq * HD + g * HD;
-  const u16* vq_base = a.qkv + (a.nq + a.nkv) * HD + g * HD;
+  // this call's K and V rows: the projection's, or (WIN) the caller's own, rotated (fdllm_attn_inplace)
+  const int ldw = WIN ? a.nkv * HD : a.ldq;
+  const u16* kq_base = (WIN ? a.kwin : a.qkv + a.nq * HD) + g * HD;
+  const u16* vq_base = (WIN ? a.vwin : a.qkv + (a.nq + a.nkv) * HD) + g * HD;
 #pragma unroll
   for (int it = 0; it < KIT; ++it) {
     const int item = tid + it * NT;
@@ -376,10 +378,10 @@ __device__ __forceinline__ void attn_chunk_load(const AttnP& a, int by, int bz, 
     key = key < kend ? key : kbeg;
     const bool win = key >= a.ws && key < a.ws + a.rows;
     if (win) {
-      const u16* src = kq_base + (size_t)(key - a.ws) * a.ldq;
+      const u16* src = kq_base + (size_t)(key - a.ws) * ldw;
       R.klo[it] = ld16<false>(src + 8 * p);
       R.khi[it] = ld16<false>(src + 64 + 8 * p);
-      if constexpr (WCS) {
+      if constexpr (WCS && !WIN) {
         const float* cs = a.rope + (size_t)(key - a.ws) * 128 + 16 * p;
 #pragma unroll
         for (int c = 0; c < 4; ++c) R.kcs[it][c] = *reinterpret_cast<const f32x4*>(cs + 4 * c);
@@ -400,7 +402,7 @@ __device__ __forceinline__ void attn_chunk_load(const AttnP& a, int by, int bz, 
       key = key < kend ? key : kbeg;
       const bool win = key >= a.ws && key < a.ws + a.rows;
       if (win) {
-        R.vv[it][qq] = ld16<false>(vq_base + (size_t)(key - a.ws) * a.ldq + 8 * dc);
+        R.vv[it][qq] = ld16<false>(vq_base + (size_t)(key - a.ws) * ldw + 8 * dc);
       } else {
         R.vv[it][qq] = *reinterpret_cast<const u32x4*>(a.vc + key * krow + g * HD + 8 * dc);
       }
@@ -408,7 +410,7 @@ __device__ __forceinline__ void attn_chunk_load(const AttnP& a, int by, int bz, 
   }
 }
 
-template <int DT, int QPW, int KH, int CH, int MASK, bool WCS = false>
+template <int DT, int QPW, int KH, int CH, int MASK, bool WCS = false, bool WIN = false>
 __device__ __forceinline__ void attn_chunk_compute(const AttnP& a, int bx, int by, int bz, unsigned char* smem,
                                                    AttnChunkRegs<QPW, KH, CH, WCS>& R, int tid) {
   typedef AttnChunkRegs<QPW, KH, CH, WCS> Regs;
@@ -470,8 +472,10 @@ __device__ __forceinline__ void attn_chunk_compute(const AttnP& a, int bx, int b
     if (key >= kend) {
       lo = hi = u32x4{0u, 0u, 0u, 0u};
     } else if (key >= a.ws && key < a.ws + a.rows) {
-      if constexpr (WCS) rope_pairs<DT>(lo, hi, R.kcs[it]);
-      else rope_tab<DT>(lo, hi, a.rope + (size_t)(key - a.ws) * 128 + 16 * p);
+      if constexpr (!WIN) {
+        if constexpr (WCS) rope_pairs<DT>(lo, hi, R.kcs[it]);
+        else rope_tab<DT>(lo, hi, a.rope + (size_t)(key - a.ws) * 128 + 16 * p);
+      }
       if (writer) {
         u16* dst = a.kc + key * krow + g * HD;
         *reinterpret_cast<u32x4*>(dst + 8 * p) = lo;
@@ -649,12 +653,12 @@ __device__ __forceinline__ void attn_chunk_compute(const AttnP& a, int bx, int b
   }
 }
 
-template <int DT, int QPW, int KH, int CH, int MASK>
+template <int DT, int QPW, int KH, int CH, int MASK, bool WIN = false>
 __device__ __forceinline__ void attn_chunk_body(const AttnP& a, int bx, int by, int bz, unsigned char* smem) {
   AttnChunkRegs<QPW, KH, CH, true> R;
   attn_chunk_qload<QPW, KH, CH, true>(a, bx, by, R, threadIdx.x);
-  attn_chunk_load<QPW, KH, CH, true>(a, by, bz, R, threadIdx.x);
-  attn_chunk_compute<DT, QPW, KH, CH, MASK, true>(a, bx, by, bz, smem, R, threadIdx.x);
+  attn_chunk_load<QPW, KH, CH, true, WIN>(a, by, bz, R, threadIdx.x);
+  attn_chunk_compute<DT, QPW, KH, CH, MASK, true, WIN>(a, bx, by, bz, smem, R, threadIdx.x);
 }
 
 // Batched call: the view of sequence b (its rows, cache, window and split partials) in a, a copy of the
@@ -683,15 +687,16 @@ __host__ __device__ __forceinline__ int attn_chunk_grid_1seq(int qg, int nkv, in
   return (nkv * S + 7) / 8 * 8 * qg;
 }
 
-template <int DT, int QPW, int KH, int CH, int MASK>
+// WIN: one sequence's rotated queries and K/V rows given by the caller (AttnP::kwin, vwin; rope null).
+template <int DT, int QPW, int KH, int CH, int MASK, bool WIN = false>
 __global__ __launch_bounds__(64 * QPW * KH) void attn_chunk_kernel(AttnP p) {
   extern __shared__ __align__(16) unsigned char smem[];
-  if (p.nseq <= 1) {
+  if (WIN || p.nseq <= 1) {
     const int QT = ((p.nq / p.nkv) * p.rows + 15) / 16, qg = (QT + QPW - 1) / QPW;
     const int i = blockIdx.x, round = i >> 3;
     const int pair = (round / qg) * 8 + (i & 7), x = round % qg;
     if (pair >= p.nkv * p.S) return;
-    attn_chunk_body<DT, QPW, KH, CH, MASK>(p, x, pair % p.nkv, pair / p.nkv, smem);
+    attn_chunk_body<DT, QPW, KH, CH, MASK, WIN>(p, x, pair % p.nkv, pair / p.nkv, smem);
     return;
   }
   const int qg = (int)gridDim.x / p.nseq, b = (int)blockIdx.x / qg;

@@ -990,11 +990,15 @@ static int check_kv_call(const fdllm_ctx* c, int rows, int cap, int layer) {
 
 // _write_rows (runtime.py:51-60): rows [start, start + rows) of the layer's cache get k and v byte for
 // byte (a cache row is nkv x head_dim contiguous elements, so the window is one contiguous range).
-static int write_kv_rows(const fdllm_ctx* c, const void* k, const void* v, int rows, void* kc, void* vc, int cap,
-                         int layer, int64_t start, hipStream_t st) {
+static int check_kv_window(int rows, int cap, int64_t start) {
   if (start < 0 || start + rows > cap)
     return fail(FDLLM_EINVAL, "KV write [%lld, %lld) outside cache capacity %d", (long long)start,
                 (long long)(start + rows), cap);
+  return FDLLM_OK;
+}
+static int write_kv_rows(const fdllm_ctx* c, const void* k, const void* v, int rows, void* kc, void* vc, int cap,
+                         int layer, int64_t start, hipStream_t st) {
+  if (int rc = check_kv_window(rows, cap, start)) return rc;
   if (rows == 0) return FDLLM_OK;
   const size_t row = (size_t)c->cfg.num_key_value_heads * c->cfg.head_dim;
   const size_t off = ((size_t)layer * cap + (size_t)start) * row, bytes = (size_t)rows * row * sizeof(uint16_t);
@@ -1019,8 +1023,8 @@ int fdllm_kv_write(fdllm_ctx* c, const void* k, const void* v, int rows, void* k
 // fast_dllm.attn_inplace (runtime.py:63-73): the write of _write_rows, then attention of the given
 // (already rotated) queries over cache rows [0, prefix_len + attend_rel) with no mask (_attend,
 // runtime.py:30-48).  The chunk kernel and attn_seq_kernel take the queries from q (AttnP::rope null: no
-// RoPE, and ws = Lk: no rows of the call are read from q's buffer or appended, the cache already holds
-// them); the prefill kernels (1024 rows and more) read rotated queries from the output buffer, where they
+// RoPE); the chunk kernel also takes and writes the K/V rows, the others find them in the cache (ws = Lk: no
+// rows of the call are read from q's buffer or appended); the prefill kernels (1024 rows and more) read rotated queries from the output buffer, where they
 // are copied first.
 int fdllm_attn_inplace(fdllm_ctx* c, const void* q, const void* k, const void* v, int rows, void* k_cache,
                        void* v_cache, int cap, int layer, int64_t prefix_len, int write_rel, int attend_rel, void* out,
@@ -1035,7 +1039,7 @@ int fdllm_attn_inplace(fdllm_ctx* c, const void* q, const void* k, const void* v
     return fail(FDLLM_EINVAL, "KV write [%lld, %lld) past the attended rows [0, %lld)", (long long)write_start,
                 (long long)(write_start + rows), (long long)attend_len);
   const hipStream_t st = (hipStream_t)stream;
-  rc = write_kv_rows(c, k, v, rows, k_cache, v_cache, cap, layer, write_start, st);
+  rc = check_kv_window(rows, cap, write_start);
   if (rc || rows == 0) return rc;
   // the reference attends over the slice k_cache[layer, :, :attend_len], which stops at the capacity
   const int Lk = (int)std::min<int64_t>(attend_len, cap);
@@ -1049,6 +1053,17 @@ int fdllm_attn_inplace(fdllm_ctx* c, const void* q, const void* k, const void* v
   a.ldq = f.num_attention_heads * f.head_dim;
   a.rope = nullptr;
   a.out = (uint16_t*)out;
+  if (attn_takes_window(a) && ((uintptr_t)k | (uintptr_t)v) % 16 == 0) {
+    // the chunk kernel takes the rows from k and v and writes them to the cache itself (its first query-tile
+    // group): one launch less than the copy before it
+    a.ws = (int)write_start;
+    a.kwin = (const uint16_t*)k;
+    a.vwin = (const uint16_t*)v;
+    HIPCHK(launch_attention(f.dtype, a, st));
+    return FDLLM_OK;
+  }
+  rc = write_kv_rows(c, k, v, rows, k_cache, v_cache, cap, layer, write_start, st);
+  if (rc) return rc;
   if (a.seq_attn) {
     a.qrot = (uint16_t*)q;  // read only: the pass that would write them is skipped
     a.ldqr = a.ldq;

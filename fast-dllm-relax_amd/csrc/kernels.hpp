@@ -208,8 +208,10 @@ struct AttnP {
   const uint16_t* qkv; int ldq;       // [rows][ldq]: q | k | v, bias added, before RoPE
   int rows, nq, nkv;
   const float* rope;                  // [rows][64][2] RoPE (cos, sin) of row r (position pos_offset + r), model-dtype values;
-                                      // null (chunk and loop kernels): the queries arrive rotated and ws >= Lk (no rows taken
-                                      // from qkv or appended)
+                                      // null: the queries arrive rotated, and ws >= Lk (no rows taken from qkv or appended) or
+                                      // kwin / vwin are set
+  // chunk kernel: this call's rotated K and its V rows, [rows][nkv * 128], instead of qkv's (null: qkv's)
+  const uint16_t* kwin; const uint16_t* vwin;
   uint16_t* kc; uint16_t* vc;         // this layer's cache [cap][nkv][128]
   int ws;                             // rows [ws, ws + rows) are this call's: taken from qkv, written to the cache
   int Lk;                             // attended keys [0, Lk)
@@ -260,6 +262,8 @@ bool attn_takes_roped(const AttnP& a);
 // the splits need (0 without splits).
 size_t plan_seq_units(AttnP& a, int ncu);
 hipError_t launch_attention(int dt, const AttnP& a, hipStream_t st);
+// whether launch_attention runs the chunk kernel for a, the one that takes kwin / vwin
+bool attn_takes_window(const AttnP& a);
 // only the RoPE and the append of the call's K/V rows (rope_kv_kernel; one sequence)
 hipError_t launch_rope_kv(int dt, const AttnP& a, hipStream_t st);
 size_t attn_partial_floats(const AttnP& a);

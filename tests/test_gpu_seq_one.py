@@ -122,3 +122,36 @@ def test_noalloc_past_the_chunk_kernels_keys():
                                                    torch.cuda.current_stream().cuda_stream))
     for a, b in ((out, want), (kc, k), (vc, v)):
         np.testing.assert_array_equal(a.float().cpu().numpy(), b.float().cpu().numpy())
+
+
+@pytest.mark.parametrize("prefix", [0, 57, 2048])
+def test_callback_rows_written_by_the_chunk_kernel(prefix):
+    """fdllm_attn_inplace on the chunk kernel, which takes the K/V rows from the caller's tensors and writes them
+    to the cache: the bytes of the rows (NaN payloads and signed zeros included), nothing beside them, and the
+    output of the same call on rows that are not 16-byte aligned (copied first)."""
+    vm = _vm(HEADS12, "bfloat16")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(23)
+    for rows in (1, 8, 17, 32):
+        cap = prefix + rows + 5
+        rnd = lambda *s: torch.randn(s, device="cuda", generator=g).bfloat16()  # noqa: E731
+        q, k, v = rnd(1, rows, 12, 128), rnd(1, rows, 2, 128), rnd(1, rows, 2, 128)
+        kc, vc = rnd(2, 1, cap, 2, 128), rnd(2, 1, cap, 2, 128)
+        log(f"case: callback of {rows} rows at {prefix}")
+        res = []
+        for shift in (0, 1):
+            kk, vv = kc.clone(), vc.clone()
+            ks = torch.empty(k.numel() + 8, dtype=k.dtype, device="cuda")[shift:shift + k.numel()].view(k.shape).copy_(k)
+            vs = torch.empty(v.numel() + 8, dtype=v.dtype, device="cuda")[shift:shift + v.numel()].view(v.shape).copy_(v)
+            out = vm.attn_inplace(q, ks, vs, kk, vv, 1, prefix, 0, rows)[2]
+            for got, rows_in, before in ((kk, k, kc), (vv, v, vc)):
+                want = before.clone()
+                want[1, 0, prefix:prefix + rows] = rows_in[0]
+                assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (rows, shift)
+            res.append(out)
+        assert torch.equal(res[0].view(torch.int16), res[1].view(torch.int16)), rows
+        special = k.view(torch.int16).clone()
+        special[0, 0, 0, :4] = torch.tensor([0x7FC1, -0x8000, -0x0041, 0x7F80], dtype=torch.int16)
+        kk, vv = kc.clone(), vc.clone()
+        vm.attn_inplace(q, special.view(torch.bfloat16), v, kk, vv, 0, prefix, 0, rows)
+        assert torch.equal(kk[0, 0, prefix:prefix + rows].view(torch.int16), special[0]), rows
