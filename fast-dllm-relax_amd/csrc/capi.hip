@@ -303,17 +303,21 @@ int run_lm_head(fdllm_ctx* c, const uint16_t* hidden, int rows, float* logits, b
   return run_gemm(c, CFG_LM_HEAD, a, 1, st);
 }
 
-// RoPE table of `rows` rows, row r at position pos[r / rows_per_seq] + r % rows_per_seq, shared by every
-// layer of the call.
-int rope_table(fdllm_ctx* c, int rows, const int32_t* pos, int rows_per_seq, hipStream_t st) {
+// The start of a call of `rows` input rows x (launch_begin_rows): the residual stream with its row statistics, the
+// RoPE table, row r at position pos[r / rows_per_seq] + r % rows_per_seq, and with nw the rows normalised by it
+// into c->xn (xblk: in fragment blocks).
+int begin_rows(fdllm_ctx* c, const void* x, int rows, bool frag, const int32_t* pos, int rows_per_seq, const uint16_t* nw,
+               int xblk, hipStream_t st) {
+  const fdllm_config& f = c->cfg;
   int rc = ensure_floats(&c->rope, &c->rope_floats, (size_t)rows * 128);
   if (rc) return rc;
-  HIPCHK(launch_rope_table(c->cfg.dtype, pos, rows, rows_per_seq, (float)(-std::log((double)c->cfg.rope_theta)),
-                           c->rope, st));
+  HIPCHK(launch_begin_rows(f.dtype, (const uint16_t*)x, rows, f.hidden_size, c->h, c->ssq, c->ws_rows, frag, pos, rows_per_seq,
+                           (float)(-std::log((double)f.rope_theta)), c->rope, nw, f.rms_norm_eps, nw ? c->xn : nullptr,
+                           xblk, st));
   return FDLLM_OK;
 }
 
-// The attention launch of the call's rows, planned into a; the RoPE table (rope_table) must hold the
+// The attention launch of the call's rows, planned into a; the RoPE table (begin_rows) must hold the
 // call's positions.  With sb, the rows are sb->nseq sequences of sb->rows (ws and Lk are then ignored).
 int plan_attention(fdllm_ctx* c, AttnP& a, int rows, uint16_t* kc, uint16_t* vc, int ws, int Lk, int mask,
                    const float* bias, long long bias_ld, const SeqBatch* sb, bool frag) {
@@ -419,7 +423,7 @@ LayerGemms layer_gemms(const fdllm_ctx* c, const Layer& L, int rows, bool frag) 
 }
 
 // Whether a call of `rows` rows runs every projection in the one-shot register-fragment body, so that its
-// activations can stay in MFMA-fragment order from load_rows to the final norm.
+// activations can stay in MFMA-fragment order from the call's start to the final norm.
 bool frag_chain(const fdllm_ctx* c, int rows) {
   if (!c->frag_on || rows > 32) return false;
   LayerGemms g = layer_gemms(c, c->layers[0], rows, false);
@@ -446,14 +450,20 @@ int run_layers(fdllm_ctx* c, const void* x_in, int rows, uint16_t* kbase, uint16
   const int ssq_ld = c->ws_rows;
   // batched calls keep the activations row-major
   const bool frag = sb == nullptr && frag_chain(c, rows);
-  HIPCHK(launch_load_rows(f.dtype, (const uint16_t*)x_in, rows, H, c->h, c->ssq, ssq_ld, st, frag));
-  int rc = rope_table(c, rows, pos_dev, sb ? sb->rows : rows, st);
-  if (rc) return rc;
-  if (frag) ++c->frag_calls;
-  // xn_ready: the previous layer's down launch also normalised this layer's qkv input into c->xn
-  // (run_resid_fused), in the layout the qkv launch takes; final_done: the last one wrote out
+  // xn_ready: this layer's qkv input is normalised in c->xn, in the layout its launch takes (the start of the
+  // call, or the previous layer's down launch: run_resid_fused); final_done: the last one wrote out
   bool xn_ready = false, final_done = false;
   int xn_layout = 0;
+  if (!frag) {
+    GemmP tq = layer_gemms(c, c->layers[0], rows, false).q;
+    const GemmPlan pq = gemm_plan(CFG_QKV, tq, 1, c->mm);
+    xn_ready = pq.kind == GK_MM;
+    xn_layout = gemm_takes_blocks(pq) ? 2 : 0;
+  }
+  int rc = begin_rows(c, x_in, rows, frag, pos_dev, sb ? sb->rows : rows, xn_ready ? c->layers[0].ln_in : nullptr,
+                      xn_layout == 2, st);
+  if (rc) return rc;
+  if (frag) ++c->frag_calls;
   for (int l = 0; l < f.num_hidden_layers; ++l) {
     const Layer& L = c->layers[l];
     uint16_t* kc = kbase + (size_t)l * layer_stride;
@@ -1247,7 +1257,7 @@ int fdllm_bench_op(fdllm_ctx* c, int op, int rows, int layer, int iters, void* k
       case FDLLM_OP_DOWN: rc = run_gemm(c, CFG_DOWN, g.d, g.dsplit, st); break;
       case FDLLM_OP_ATTENTION:
         // the block's rows sit at the end of the attended range, as in a full cached step
-        if (it == 0) rc = rope_table(c, rows, c->zero_i32, rows, st);
+        if (it == 0) rc = begin_rows(c, c->h, rows, false, c->zero_i32, rows, nullptr, 0, st);
         if (rc == FDLLM_OK)
           rc = run_attention(c, rows, (uint16_t*)k + li * stride, (uint16_t*)v + li * stride, attend_len - rows,
                              attend_len, 0, nullptr, 0, st, nullptr, frag);

@@ -183,13 +183,13 @@ hipError_t launch_unmask(const int32_t* ids, const float* maxp, const UnmaskP& u
 hipError_t launch_kv_copy(const void* k, const void* v, void* kd, void* vd, size_t bytes, hipStream_t st);
 hipError_t launch_embed(const int32_t* ids, int n, const uint16_t* table, int vocab, int hidden, uint16_t* out,
                         hipStream_t st);
-// copy the input rows into the residual stream and emit their per-16-column sums of squares; hfrag: h
-// in MFMA-fragment order (rows <= 32)
-hipError_t launch_load_rows(int dt, const uint16_t* x, int rows, int hidden, uint16_t* h, float* ssq, int ssq_ld,
-                            hipStream_t st, int hfrag = 0);
-// RoPE (cos, sin) table: row r sits at position pos_offset[r / rows_per_seq] + r % rows_per_seq
-hipError_t launch_rope_table(int dt, const int32_t* pos_offset, int rows, int rows_per_seq, float neg_log_theta,
-                             float* tab, hipStream_t st);
+// The start of a call: the input rows copied into the residual stream h (hfrag: in MFMA-fragment order, rows <= 32)
+// with their per-16-column sums of squares; the RoPE (cos, sin) table, row r at position pos_offset[r /
+// rows_per_seq] + r % rows_per_seq; and with y the first layer's normalised rows (weight w; yblk: in the
+// large-M kernels' fragment blocks).  hidden at most 2048.
+hipError_t launch_begin_rows(int dt, const uint16_t* x, int rows, int hidden, uint16_t* h, float* ssq, int ssq_ld, int hfrag,
+                             const int32_t* pos_offset, int rows_per_seq, float neg_log_theta, float* tab,
+                             const uint16_t* w, float eps, uint16_t* y, int yblk, hipStream_t st);
 // y = RMSNorm(h) from the sums of squares the producer left (final norm); hfrag: h in MFMA-fragment order;
 // yblk: y in the large-M kernel's fragment blocks (frag_blk_off) instead of row-major
 hipError_t launch_norm_rows(int dt, const uint16_t* h, int rows, int hidden, const float* ssq, int ssq_ld,

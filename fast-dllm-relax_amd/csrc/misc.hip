@@ -1,4 +1,4 @@
-// Row kernels of the cached step: embedding gather, residual-stream load, final RMSNorm.
+// Row kernels of the cached step: embedding gather, the start of a call, RMSNorm.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -14,35 +14,6 @@ __global__ __launch_bounds__(256) void embed_kernel(const int32_t* ids, const u1
   const u32x4* src = reinterpret_cast<const u32x4*>(table + (size_t)id * hidden);
   u32x4* dst = reinterpret_cast<u32x4*>(out + (size_t)r * hidden);
   for (int c = threadIdx.x; c < hidden / 8; c += blockDim.x) dst[c] = src[c];
-}
-
-// The residual stream h starts as a copy of the input rows; each thread of the first H / 16 also
-// leaves the sum of squares of one 16-column tile of its row for the first layer's RMSNorm (the
-// layers' own residual epilogues leave the same statistics for the next norm).
-template <int DT>
-__global__ __launch_bounds__(256) void load_rows_kernel(const u16* x, int hidden, u16* h, float* ssq, int ssq_ld,
-                                                        int hfrag) {
-  const int r = blockIdx.x;
-  const u32x4* src = reinterpret_cast<const u32x4*>(x + (size_t)r * hidden);
-  for (int c = threadIdx.x; c < hidden / 8; c += blockDim.x)
-    *reinterpret_cast<u32x4*>(h + (hfrag ? frag_off(r, 8 * c) : (size_t)r * hidden + 8 * c)) = src[c];
-  for (int t = threadIdx.x; t < hidden / 16; t += blockDim.x) {
-    const u32x4 a = src[2 * t], b = src[2 * t + 1];
-    float ss = 0.f;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float a0 = lo_f32<DT>(a[c]), a1 = hi_f32<DT>(a[c]);
-      ss += a0 * a0;
-      ss += a1 * a1;
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float b0 = lo_f32<DT>(b[c]), b1 = hi_f32<DT>(b[c]);
-      ss += b0 * b0;
-      ss += b1 * b1;
-    }
-    ssq[(size_t)t * ssq_ld + r] = ss;
-  }
 }
 
 // One normalised element, w * rnd(x * inv) rounded to the model dtype.  Each element is computed on its
@@ -191,18 +162,75 @@ __global__ __launch_bounds__(NT) void resid_norm_kernel(const float* part, int s
   }
 }
 
-// RoPE tables of one call (cuda.py:288-299): position pos_offset + r, inv_freq = exp(-ln(theta) * i / 64),
-// angle = pos * inv_freq in fp32, cos / sin in fp32 rounded to the model dtype (emb = [f, f], so one
-// entry serves dims i and i + 64).  Shared by every layer's attention.
+// The start of a call, one workgroup per row r (three launches before: copy, RoPE table, first norm; each about
+// 4.7 us, which is a launch's own cost at the rows of a step):
+//   - the residual stream h starts as a copy of the input row, with the sums of squares of its 16-column tiles
+//     for the first layer's RMSNorm (the layers' own residual epilogues leave the same statistics for the next);
+//   - the RoPE table's row (cuda.py:288-299): position pos_offset + r, inv_freq = exp(-ln(theta) * i / 64), angle =
+//     pos * inv_freq in fp32, cos / sin in fp32 rounded to the model dtype (emb = [f, f], so one entry serves dims
+//     i and i + 64); shared by every layer's attention;
+//   - with y, the first layer's normalised row (norm_rows_kernel's arithmetic, from the same sums), row-major or
+//     with yblk in the large-M GEMMs' fragment blocks.
 template <int DT>
-__global__ __launch_bounds__(64) void rope_table_kernel(const int32_t* pos_offset, int rows_per_seq, float nlt,
-                                                        float* tab) {
-  const int r = blockIdx.x, i = threadIdx.x;
-  const int b = r / rows_per_seq;
-  const float pos = (float)(pos_offset[b] + (r - b * rows_per_seq));
-  const float fr = pos * expf((nlt * (float)i) / 64.0f);
-  tab[((size_t)r * 64 + i) * 2] = rnd<DT>(cosf(fr));
-  tab[((size_t)r * 64 + i) * 2 + 1] = rnd<DT>(sinf(fr));
+__global__ __launch_bounds__(256) void begin_rows_kernel(const u16* x, int hidden, u16* h, float* ssq, int ssq_ld, int hfrag,
+                                                         const int32_t* pos_offset, int rows_per_seq, float nlt, float* tab,
+                                                         const u16* w, float eps, u16* y, int yblk) {
+  constexpr int MAXH = 2048;  // hidden sizes up to this (the launcher checks)
+  __shared__ float tss[MAXH / 16];
+  __shared__ float inv_s;
+  const int r = blockIdx.x;
+  const u32x4* src = reinterpret_cast<const u32x4*>(x + (size_t)r * hidden);
+  for (int c = threadIdx.x; c < hidden / 8; c += 256)
+    *reinterpret_cast<u32x4*>(h + (hfrag ? frag_off(r, 8 * c) : (size_t)r * hidden + 8 * c)) = src[c];
+  for (int t = threadIdx.x; t < hidden / 16; t += 256) {
+    const u32x4 a = src[2 * t], b = src[2 * t + 1];
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float a0 = lo_f32<DT>(a[c]), a1 = hi_f32<DT>(a[c]);
+      ss += a0 * a0;
+      ss += a1 * a1;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float b0 = lo_f32<DT>(b[c]), b1 = hi_f32<DT>(b[c]);
+      ss += b0 * b0;
+      ss += b1 * b1;
+    }
+    ssq[(size_t)t * ssq_ld + r] = ss;
+    tss[t] = ss;
+  }
+  if (threadIdx.x >= 192) {  // (the last wave: the first ones have the tile sums)
+    const int i = threadIdx.x - 192, b = r / rows_per_seq;
+    const float pos = (float)(pos_offset[b] + (r - b * rows_per_seq));
+    const float fr = pos * expf((nlt * (float)i) / 64.0f);
+    tab[((size_t)r * 64 + i) * 2] = rnd<DT>(cosf(fr));
+    tab[((size_t)r * 64 + i) * 2 + 1] = rnd<DT>(sinf(fr));
+  }
+  if (y == nullptr) return;
+  __syncthreads();
+  const int ntiles = hidden / 16;
+  if (threadIdx.x < 64) {
+    float pq[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v = 0.f;
+      for (int t = 64 * q + (int)threadIdx.x; t < ntiles; t += 256) v += tss[t];
+      pq[q] = 64 * q < ntiles ? wave_sum(v) : 0.f;
+    }
+    if (threadIdx.x == 0) inv_s = 1.0f / sqrtf(((pq[0] + pq[1]) + (pq[2] + pq[3])) / (float)hidden + eps);
+  }
+  __syncthreads();
+  const float inv = inv_s;
+  for (int u = threadIdx.x; u < hidden / 8; u += 256) {
+    const u32x4 hv = src[u], wv = *reinterpret_cast<const u32x4*>(w + 8 * u);
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = pack2(norm_elem<DT>(lo_f32<DT>(wv[e]), lo_f32<DT>(hv[e]), inv),
+                   norm_elem<DT>(hi_f32<DT>(wv[e]), hi_f32<DT>(hv[e]), inv));
+    *reinterpret_cast<u32x4*>(y + (yblk ? frag_blk_off(r, 8 * u, hidden / 32) : (size_t)r * hidden + 8 * u)) = o;
+  }
 }
 
 // The cache write of fast_dllm.kv_write / attn_inplace (_write_rows, fast_dllm_relax/runtime.py:51-60):
@@ -230,24 +258,13 @@ hipError_t launch_embed(const int32_t* ids, int n, const uint16_t* table, int vo
   return hipGetLastError();
 }
 
-hipError_t launch_load_rows(int dt, const uint16_t* x, int rows, int hidden, uint16_t* h, float* ssq, int ssq_ld,
-                            hipStream_t st, int hfrag) {
-  if (hfrag && rows > 32) return hipErrorInvalidValue;
-  if (dt == DT_BF16)
-    hipLaunchKernelGGL(load_rows_kernel<DT_BF16>, dim3(rows), dim3(256), 0, st, x, hidden, h, ssq, ssq_ld, hfrag);
-  else
-    hipLaunchKernelGGL(load_rows_kernel<DT_F16>, dim3(rows), dim3(256), 0, st, x, hidden, h, ssq, ssq_ld, hfrag);
-  return hipGetLastError();
-}
-
-hipError_t launch_rope_table(int dt, const int32_t* pos_offset, int rows, int rows_per_seq, float neg_log_theta, float* tab,
-                             hipStream_t st) {
-  if (dt == DT_BF16)
-    hipLaunchKernelGGL(rope_table_kernel<DT_BF16>, dim3(rows), dim3(64), 0, st, pos_offset, rows_per_seq, neg_log_theta,
-                       tab);
-  else
-    hipLaunchKernelGGL(rope_table_kernel<DT_F16>, dim3(rows), dim3(64), 0, st, pos_offset, rows_per_seq, neg_log_theta,
-                       tab);
+hipError_t launch_begin_rows(int dt, const uint16_t* x, int rows, int hidden, uint16_t* h, float* ssq, int ssq_ld, int hfrag,
+                             const int32_t* pos_offset, int rows_per_seq, float neg_log_theta, float* tab,
+                             const uint16_t* w, float eps, uint16_t* y, int yblk, hipStream_t st) {
+  if ((hfrag && rows > 32) || hidden % 32 || hidden > 2048) return hipErrorInvalidValue;
+  auto kern = dt == DT_BF16 ? begin_rows_kernel<DT_BF16> : begin_rows_kernel<DT_F16>;
+  hipLaunchKernelGGL(kern, dim3(rows), dim3(256), 0, st, x, hidden, h, ssq, ssq_ld, hfrag, pos_offset, rows_per_seq,
+                     neg_log_theta, tab, w, eps, y, yblk);
   return hipGetLastError();
 }
 
