@@ -604,7 +604,7 @@ def decode_gap_events(args) -> int:
 def trace_gaps(path: str) -> int:
     """GPU idle time between model calls of the decode loop, from a rocprofv3 kernel trace (csv).
 
-    A model call starts with its first layer-loop kernel (load_rows_kernel) and ends with the confidence
+    A model call starts with its first layer-loop kernel (begin_rows_kernel) and ends with the confidence
     reduction (confidence_unmask_kernel on the device loop, confidence_combine_kernel on the host loop).
     The gap is the time from the end of one call's last kernel to the start of the next call's first,
     over the calls of the last generation in the trace (the loop's steady state); it holds whatever the
@@ -619,7 +619,7 @@ def trace_gaps(path: str) -> int:
     rows.sort()
     calls, cur = [], None
     for s, e, n in rows:
-        if "load_rows_kernel" in n:
+        if "begin_rows_kernel" in n:
             cur = [s, None, 0]
         if cur is None:
             continue

@@ -61,8 +61,8 @@ static void seq_one_splits(AttnPlan& p, int QT, int nkv, int Lk, int ncu) {
 }
 
 // Launch plan: short row blocks (the cached decode step) use attn_chunk_kernel with one key chunk of
-// CH keys per workgroup; long row blocks (prefill, stateless forward) use attn_kernel with few, long
-// key ranges per workgroup.
+// CH keys per workgroup; one sequence's longer unmasked calls attn_seq_kernel in key splits (p.seq); the
+// others attn_kernel with few, long key ranges per workgroup, or (launch_dt) attn_prefill_kernel.
 AttnPlan attn_plan(int rows, int nq, int nkv, int Lk, int target_wgs, int nseq, int mask, int ncu) {
   AttnPlan p{};
   const int QT = ((nq / nkv) * rows + 15) / 16;

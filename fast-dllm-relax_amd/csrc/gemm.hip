@@ -210,7 +210,7 @@ template <int MF, int TPW, int NWN, int KP, int D>
 struct WkCfg {
   static constexpr int mf = MF, tpw = TPW, nwn = NWN, kp = KP, d = D;
   static constexpr int bm = 16 * MF, bn_tiles = NWN * TPW, kss = KP;
-  static constexpr size_t lds_in = (size_t)(D + 1) * KP * MF * 1024, lds_red = (size_t)KP * NWN * TPW * MF * 1024;
+  static constexpr size_t lds_in = (size_t)(D + 1) * KP * MF * 1024, lds_red = (size_t)KP * NWN * TPW * (MF / 2) * 1024;
   static constexpr size_t lds = lds_in > lds_red ? lds_in : lds_red;
 };
 using WkGu4 = WkCfg<4, 2, 3, 2, 4>;  // (depth 3 to 12 and one k group measure the same, four k groups 1.5 us more)
@@ -506,13 +506,7 @@ template <int DT, int EPI, class W>
 static hipError_t launch_wk_cfg(const GemmP& a, const GemmPlan& p, hipStream_t st) {
   auto kern = gemm_wk_kernel<DT, EPI, W::mf, W::tpw, W::nwn, W::kp, W::d>;
   if (a.KS % (p.ksplit * W::kp)) return hipErrorInvalidValue;
-  static bool attr = false;  // per instantiation
-  if (!attr) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)W::lds) !=
-        hipSuccess)
-      (void)hipGetLastError();
-    attr = true;
-  }
+  static_assert(W::lds <= 64 * 1024, "no LDS attribute needed");
   const int total = p.nbm * p.nbn, per = (total + 7) / 8;
   hipLaunchKernelGGL(kern, dim3(8 * per, p.ksplit), dim3(64 * W::nwn * W::kp), W::lds, st, a, p.nbm, p.nbn);
   if (p.ksplit > 1 && !a.part_rows) {

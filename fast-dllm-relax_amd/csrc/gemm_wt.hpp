@@ -491,7 +491,7 @@ void gemm_wk_kernel(GemmP a, int nbm, int nbn) {
   constexpr int VPS = TPW + DPW;             // vector memory instructions per wave per stage
   static_assert(D >= 2 && (D - 1) * VPS < 64, "outstanding copies fit the memory counter");
   static_assert(EPI != EPI_SILU_PAIR || TPW % 2 == 0, "gate/up pairs stay within a wave");
-  static_assert(MF % KP == 0, "the groups finish as many row blocks each");
+  static_assert(KP == 2 && MF % 2 == 0, "two groups, each finishing every other row block");
   static_assert(EPI != EPI_LOGITS, "no confidence tiles here");
   extern __shared__ __align__(16) unsigned char smem[];  // [R][KP][MF][1 KB]
 
@@ -581,12 +581,12 @@ void gemm_wk_kernel(GemmP a, int nbm, int nbn) {
   __syncthreads();
 
   // the groups' sums: every wave leaves the row blocks other groups finish, and adds the others' of its own
-  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [KP][NWN][TPW][MF][64]
+  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [KP][NWN][TPW][MF / 2][64]: each wave's blocks of the other group
 #pragma unroll
   for (int j = 0; j < TPW; ++j)
 #pragma unroll
     for (int f = 0; f < MF; ++f)
-      if (f % KP != kp) red[((((size_t)kp * NWN + wn) * TPW + j) * MF + f) * 64 + lane] = acc[j][f];
+      if (f % KP != kp) red[((((size_t)kp * NWN + wn) * TPW + j) * (MF / 2) + f / 2) * 64 + lane] = acc[j][f];
   __syncthreads();
   static_for<0, KP>([&](auto kc) {
     constexpr int K0 = decltype(kc)::value;
@@ -598,7 +598,7 @@ void gemm_wk_kernel(GemmP a, int nbm, int nbn) {
         f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
-          const f32x4 v = k == K0 ? acc[j][f] : red[((((size_t)k * NWN + wn) * TPW + j) * MF + f) * 64 + lane];
+          const f32x4 v = k == K0 ? acc[j][f] : red[((((size_t)k * NWN + wn) * TPW + j) * (MF / 2) + f / 2) * 64 + lane];
           sum = k == 0 ? v : sum + v;
         }
         acc[j][f] = sum;
