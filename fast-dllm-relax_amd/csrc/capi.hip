@@ -107,8 +107,10 @@ struct fdllm_ctx {
   unsigned* attn_cnt = nullptr;  // attn_seq_kernel's arrival counters (SEQ_CNT_MAX, zero between launches)
   int fuse_down = 1;      // large-M down launches with k splits: split sum + residual + next RMSNorm in one launch
   // large-M o_proj with a forced k split and its split sum + residual + the next norm in one launch: -1 with
-  // three splits up to 256 rows (128-row batched step: 14.8 + 4.8 us norm -> 8.1 + 7.1 us; at 512 rows it
-  // measured slower, 3.88 -> 3.94 ms per step with two splits), 0 never, N > 1 with N splits at any size
+  // three or two splits up to 256 and from 513 rows, where that many of its blocks make one round of the compute
+  // units (us per layer of a prefill, two / three splits / none: 192 rows 67.6 / 67.0 / -, 200 rows 66.6 / 68.6 / -,
+  // 400 rows 88.7 / 87.9 / 87.1, 576 rows 96.4 / 98.7 / 100.1, 672 rows 115.3 / 114.5 / 114.0), 0 never, N > 1 with N
+  // splits at any size
   int fuse_oproj = -1;
   // large-M calls whose attention starts with the RoPE / KV-append pass (prefill, batched sequences): that
   // pass done by qkv's epilogue instead (FDLLM_QKV_ROPE=0: the separate pass)
@@ -502,7 +504,13 @@ int run_layers(fdllm_ctx* c, const void* x_in, int rows, uint16_t* kbase, uint16
     HIPCHK(launch_attention(f.dtype, at, st));
     // o_proj + the post-attention norm: with a forced k split, when gate_up takes normalised rows
     bool gu_ready = false;
-    const int oproj_split = c->fuse_oproj > 1 ? c->fuse_oproj : (c->fuse_oproj < 0 && rows <= 256 ? 3 : 0);
+    int oproj_split = c->fuse_oproj > 1 ? c->fuse_oproj : 0;
+    if (c->fuse_oproj < 0 && !frag && (rows <= 256 || rows > 512)) {
+      GemmP to = g.o;
+      const GemmPlan po = gemm_plan(CFG_OPROJ, to, 1, c->mm);
+      const int round = std::min(c->ncu, c->mm.target_wgs), wgs = po.kind == GK_MM ? po.nbm * po.nbn : round;
+      oproj_split = 3 * wgs <= round ? 3 : 2 * wgs <= round ? 2 : 0;
+    }
     if (!frag && oproj_split > 1) {
       MmPolicy po = c->mm;
       po.force_split = oproj_split;
