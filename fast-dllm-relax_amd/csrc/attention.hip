@@ -191,9 +191,9 @@ static hipError_t launch_chunk_mask(const AttnP& a, const AttnPlan& p, hipStream
 // four tiles alone until their workgroups pass one round of the 256 compute units by a quarter, then paired
 // (uneven blocks in a second round cost more than the pairs' fewer workgroups), all twelve alone once that
 // gives 180 workgroups and paired once the pairs give 7/8 of a round.  Measured (1.5B bf16
-// build_prefix_cache, us per layer; four alone / four paired / twelve alone / twelve paired): 509 rows 115.6 /
-// 119.3 / 123.8 / 133.4, 1500 rows 238 / 241 / 255 / 263, 2048 rows 283 / 273 / 289 / 299, 3000 rows 411 / 419 /
-// 407 / 416, 6000 rows 783 / 805 / 719 / 724, 8192 rows 1081 / 1055 / 963 / 949.
+// build_prefix_cache, us per layer; four alone / four paired / twelve alone / twelve paired): 509 rows 109.8 /
+// 113.7 / 119.2 / 128.2, 1500 rows 226 / 229 / 245 / 254, 2048 rows 271 / 261 / 282 / 291, 3000 rows 386 / 397 /
+// 389 / 398, 4096 rows 494 / 489 / 481 / 487, 6000 rows 762 / 787 / 708 / 716, 8192 rows 1041 / 1025 / 942 / 932.
 constexpr int PREFILL_ALONE_MAX_WGS = 320, PREFILL_WHOLE_MIN_WGS = 180, PREFILL_WHOLE_PAIRED_MIN_WGS = 224;
 
 template <int DT, int MASK, int TQ>

@@ -838,14 +838,14 @@ __global__ __launch_bounds__(128) void rope_kv_kernel(AttnP p) {
 }
 
 // One block of an online softmax over a lane's 4 N raw scores s of its query (the query's other keys sit in
-// lanes l ^ 16, l ^ 32, l ^ 48): s becomes p = 2^(s c2 - m) with m the query's reference, l the lane's part of
-// the sum of p (its four lanes' parts are added once, at the end), o the accumulator.  The reference is a
-// maximum seen so far that is renewed only when a score passes it by more than 2^LAZY_MAX: p is then at
-// most 2^8, a power of two off the usual p <= 1 and as exact (fp32, and its rounding to the model dtype,
-// are relative; fp16 holds 2^8 and loses fewer small p), and most blocks have no reduction across lanes
-// and no rescaling.  Scale and subtraction are one fma, so per score: fma, exp2, add, half a max and half a
-// rounding.
-constexpr float LAZY_MAX = 8.0f;
+// lanes l ^ 16, l ^ 32, l ^ 48): s becomes p = 2^(s c2 - m) with m the query's running maximum, l the lane's part of
+// the sum of p (its four lanes' parts are added once, at the end), o the accumulator.  Blocks without a new
+// maximum for any of the wave's queries have no reduction across lanes and no rescaling.  The maximum is never
+// left behind: that keeps each row's largest p at 1, which the model dtype holds exactly.  (Renewed only once
+// passed by 2^8, the attention of 8192 rows took 209 us instead of 238, but the largest p's own rounding reached the
+// output: scores of deviation 3 over 2048 keys, relative error against float64 2.16e-3 instead of 1.74e-3 in
+// bfloat16, 2.70e-4 instead of 2.17e-4 in float16.)
+// Scale and subtraction are one fma, so per score: fma, exp2, add, half a max and half a rounding.
 
 // two probabilities rounded to the model dtype: 2^x is no product, so fp16 needs none of pack_f32x2's care
 // about mixed-precision fmas (whose empty asm keeps the values in registers of their own)
@@ -854,14 +854,14 @@ template <int DT> __device__ __forceinline__ uint32_t pack_p(float a, float b) {
   else return pack2(f32_to_f16(a), f32_to_f16(b));
 }
 template <int N, int NO>
-__device__ __forceinline__ void lazy_softmax(f32x4 (&s)[N], float c2, float& m, float& l, f32x4 (&o)[NO]) {
+__device__ __forceinline__ void block_softmax(f32x4 (&s)[N], float c2, float& m, float& l, f32x4 (&o)[NO]) {
   float mx = s[0][0];
 #pragma unroll
   for (int kt = 0; kt < N; ++kt)
 #pragma unroll
     for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[kt][e]);
   mx *= c2;
-  if (__builtin_amdgcn_ballot_w64(mx > m + LAZY_MAX) != 0) {
+  if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
     const float m_new = fmaxf(m, rows_max(mx));
     const float alpha = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.f : m_new));
     l *= alpha;
@@ -890,7 +890,7 @@ __device__ __forceinline__ void lazy_softmax(f32x4 (&s)[N], float c2, float& m, 
 // second 64 keys of every 128-key stage.  Two waves per SIMD, so that one's softmax (VALU) runs while the
 // other's MFMAs do: with four waves and no key parts a stage's MFMAs (1536 cycles of a SIMD), softmax
 // (about 1900) and LDS waits followed one another (per layer at 8192 / 2048 / 509 rows: 317 / 50 / 14.4 us with
-// one wave per SIMD, 277 / 41.6 us with lazy_softmax as well, 212 / 35 / 10.7 us with both; 1.0 PFLOP/s at 8192).
+// one wave per SIMD, 238 / 36.7 / 11.0 us with two; 0.87 PFLOP/s at 8192).
 // The parts of a query block are merged through LDS when its keys end (part 0 + part 1, each relative to the
 // larger maximum).  MFMAs and VALU work now bound it, about equally.
 //
@@ -1099,7 +1099,7 @@ void attn_prefill_kernel(AttnP a, int paired) {
           for (int e = 0; e < 4; ++e)
             s[i][kt][e] = k0 + 16 * kt + 4 * lg + e < kend_q[i] ? s[i][kt][e] : -INFINITY;
       }
-      lazy_softmax(s[i], c2, m_run[i], l_run[i], o[i]);
+      block_softmax(s[i], c2, m_run[i], l_run[i], o[i]);
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
         pb[i][ks] = u32x4{pack_p<DT>(s[i][2 * ks][0], s[i][2 * ks][1]),

@@ -43,6 +43,36 @@ def test_prefill_attention_unmasked(monkeypatch, kw, form, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("hpw", [0, 6], ids=["4 tiles", "12 tiles"])
+def test_prefill_attention_peaked_rows(monkeypatch, hpw, dtype):
+    """Each row's largest probability is exact: it is 2^0 against the running maximum, so its rounding to the model
+    dtype for P.V costs nothing.  One key holds all the weight that reaches the output (the other keys' V rows are
+    zero) with a score up to 2^12 past the zero scores before it: o = w v, and its only rounding is the output's.
+    Half an ulp of the result, and 2 percent of that for the fp32 sums (about 40 roundings of 2^-24 against
+    float16's half ulp of at least 2^-12)."""
+    vm = _vm(HEADS12, dtype, monkeypatch, {"FDLLM_PREFILL_PAIR": "0", "FDLLM_PREFILL_HPW": str(hpw)})
+    td, nq, nkv, L, rows = TORCH_DTYPES[dtype], 12, 2, HEADS12["num_hidden_layers"], 1024
+    g = torch.Generator(device="cuda")
+    g.manual_seed(14)
+    c2 = 1.4426950408889634 / 128 ** 0.5
+    for peak in (40, 100, 900, 1023):  # the peak in either key part of the first stage, and of later ones
+        lag = torch.rand((1, rows, nq), device="cuda", generator=g) * 12
+        q = torch.zeros((1, rows, nq, 128), dtype=td, device="cuda")
+        q[..., 5] = (lag / c2 / 8).to(td)
+        k, v = (torch.zeros((1, rows, nkv, 128), dtype=td, device="cuda") for _ in range(2))
+        k[:, peak, :, 5] = 8
+        v[:, peak] = (0.5 + torch.rand((nkv, 128), device="cuda", generator=g)).to(td)
+        kc = torch.zeros((L, 1, rows, nkv, 128), dtype=td, device="cuda")
+        log(f"case: peak at key {peak} of {rows}, {6 if hpw == 6 else 2} heads per workgroup, {dtype}")
+        _, _, out = vm.attn_inplace(q, k, v, kc, torch.zeros_like(kc), 0, 0, 0, rows)
+        lead = torch.exp2(q[0, :, :, 5].double() * 8 * c2)
+        want = (lead / (lead + (rows - 1)))[..., None] * v[0, peak].double().repeat_interleave(nq // nkv, 0)
+        half_ulp = torch.exp2(torch.floor(torch.log2(want)) - (8 if dtype == "bfloat16" else 11))
+        worst = float(((out[0].double() - want).abs() / half_ulp).max())
+        assert worst < 1.02, (peak, worst)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 def test_prefill_attention_block_causal(dtype):
     """The block-causal rule as a key bound against the same rule as an explicit bias (attn_kernel)."""
     vm = _vm(TINY, dtype)
