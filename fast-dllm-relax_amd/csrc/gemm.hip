@@ -147,12 +147,6 @@ GemmShape gemm_shape(int cfg) {
   return GemmShape{l, 0};
 }
 
-// rows from which the lm_head (with its confidence statistics) takes the register-weight kernel (us per
-// launch with the statistics, fp16, register-weight / 64 x 256 LDS-staged blocks: 199 / 228-232 at 256 rows,
-// 326 / 386 at 512, even at 112-128)
-#ifndef FD_WR_LM_MIN_ROWS
-#define FD_WR_LM_MIN_ROWS 256
-#endif
 // stages in flight of the register-weight kernel
 #ifndef FD_WR_DEPTH
 #define FD_WR_DEPTH 3
@@ -216,99 +210,14 @@ struct WkCfg {
 using WkGu4 = WkCfg<4, 2, 3, 2, 4>;  // (depth 3 to 12 and one k group measure the same, four k groups 1.5 us more)
 using WkGu6 = WkCfg<6, 2, 3, 2, 4>;
 using WkGu8 = WkCfg<8, 2, 3, 2, 3>;
-enum MmId : int { MM_SMALL = 0, MM_WIDE = 1, MM_WIDE_D = 2, MM_BIG = 3, MM_WT = 4, MM_WR = 5, MM_WR_S = 6, MM_WR_M = 7, MM_WR_T = 8, MM_WR_3 = 9, MM_WT_8 = 10, MM_WT_256 = 11, MM_WK_GU4 = 12, MM_WK_GU6 = 13, MM_WK_GU8 = 14 };
-struct MmInfo { int bm, bn_tiles, kss; };
-template <class M> constexpr MmInfo mm_info_of() { return MmInfo{M::bm, M::bn_tiles, M::kss}; }
-static MmInfo mm_info(int id) {
-  switch (id) {
-    case MM_WIDE: return mm_info_of<MmWide>();
-    case MM_WIDE_D: return mm_info_of<MmWideD>();
-    case MM_BIG: return mm_info_of<MmBig>();
-    case MM_WT: return mm_info_of<WtBig>();
-    case MM_WR: return mm_info_of<WrBig>();
-    case MM_WR_S: return mm_info_of<WrSmall>();
-    case MM_WR_M: return mm_info_of<WrMid>();
-    case MM_WR_T: return mm_info_of<WrTiny>();
-    case MM_WR_3: return mm_info_of<WrB3>();
-    case MM_WT_8: return mm_info_of<WtBig8>();
-    case MM_WT_256: return mm_info_of<WtB256>();
-    case MM_WK_GU4: return mm_info_of<WkGu4>();
-    case MM_WK_GU6: return mm_info_of<WkGu6>();
-    case MM_WK_GU8: return mm_info_of<WkGu8>();
-    default: return mm_info_of<MmSmall>();
-  }
+// mm_choice.hpp plans with these blocks' sizes
+template <class M> constexpr bool mm_is(int id) {
+  return mm_info(id).bm == M::bm && mm_info(id).bn_tiles == M::bn_tiles && mm_info(id).kss == M::kss;
 }
-// Rows from which a projection takes the register-weight kernel by default.  Measured (1.5B, us per
-// launch, register-weight / previous kernel): gate_up 53 / 47 at 512 rows, 110 / 118 at 2048, 377 / 448
-// at 8192; down 40 / 30, 79 / 80, 189 / 192; qkv 37 / 31 at 2048, 75 / 106 at 8192; o_proj 38 / 23,
-// 57 / 70.  Below these sizes its 128 x 256 blocks leave too few workgroups without a k split.
-static int wr_default_min_rows(int cfg) {
-  if (cfg == CFG_LM_HEAD) return FD_WR_LM_MIN_ROWS;
-  return cfg == CFG_GATE_UP || cfg == CFG_DOWN ? 2048 : 4096;
-}
-static int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
-  // The large blocks by how their counts fill the 256 compute units (two workgroups each), us per launch.
-  // Register-weight 128 x 256 gate_up of 641 to 896 rows, one round of at most 490 blocks / LDS-staged: 50.7 /
-  // 56.7 at 660 rows, 51.7 / 59.4 at 896 (but 51.3 / 43.9 at 640, 68.3 / 59.1 at 900).  o_proj past 2560 rows, where
-  // its 64 x 128 blocks start a second round: register-weight 128 x 192 / 64 x 128: 28.6 / 36.0 at 2700, 28.8 / 36.7
-  // at 3000 (28.5 / 23.9 at 2560).  Down, register-weight 128 x 192 / LDS-staged: 31.9 / 33.8 at 680 rows, 37.6 / 40.3
-  // at 896, 39.4 / 41.3 at 1024, 55.5 / 52.5 at 1100, 59.9 / 59.4 at 1400, 61.7 / 64.1 at 1600, 101 / 97 at 2800, 98 / 105
-  // at 3500; 128 x 256 where their splits come to one round, 47.8 / 53.4 at 1200, 78.6 / 86.9 at 2100, 79.4 / 90.1 at 2400.
-  if (pol.wr_min_rows == 0 && ((pol.wr_ops >> cfg) & 1) && pol.wr_ffn < 0) {
-    const bool b3 = pol.wr3 && ntiles % WrB3::bn_tiles == 0;
-    if (cfg == CFG_GATE_UP && M > 640 && M <= 896) return MM_WR;
-    if (cfg == CFG_OPROJ && M > 2560 && b3) return MM_WR_3;
-    if (cfg == CFG_DOWN && ((M > 1024 && M <= 1280) || (M > 2048 && M <= 2560))) return MM_WR;
-    if (cfg == CFG_DOWN && ((M > 672 && M <= 1024) || (M > 1536 && M <= 2048)) && b3) return MM_WR_3;
-    if (cfg == CFG_DOWN && M > 2560 && M <= 3200 && ntiles % WtBig::bn_tiles == 0) return MM_WT;
-  }
-  const int min_rows = pol.wr_min_rows > 0 ? pol.wr_min_rows : wr_default_min_rows(cfg);
-  if (M >= std::max(min_rows, 33) && ((pol.wr_ops >> cfg) & 1))
-    return pol.wr3 && (cfg == CFG_OPROJ || cfg == CFG_DOWN) && ntiles % WrB3::bn_tiles == 0 ? MM_WR_3 : MM_WR;
-  // qkv and o_proj below that: 64 x 128 register-weight blocks (us per launch, qkv including its norm pass,
-  // against the LDS-staged 64 x 128 kernel): qkv 16.2 / 14.9 at 128 rows, 23.2 / 20.2 at 512, 26.2 / 19.4
-  // at 1024, 30.8 / 28.6 at 2048; o_proj 15.2 / 14.0 at 384, 15.4 / 14.0 at 512, 19.3 / 15.1 at 1024, but
-  // 23.3 / 26.4 at 2048 (equal below 384).  Up to 512 rows 64 x 64 blocks, twice the workgroups, do better
-  // still (us, 64 x 128 / 64 x 64 blocks): qkv 14.4 / 13.4 at 128 rows, 15.7 / 13.7 at 256, 16.8 / 14.9 at
-  // 512 (but 19.4 / 21.2 at 1024); o_proj 12.8 / 11.9, 12.8 / 11.9, 14.0 / 12.0 (15.1 / 21.4 at 1024)
-  // o_proj up to 1344 rows, one round of 64 x 128 blocks (16.1 / 20.0 at 1300 rows, 25.9 / 23.3 at 1500)
-  if (M >= 33 && ((pol.wr_small_ops >> cfg) & 1) && (cfg == CFG_QKV || (cfg == CFG_OPROJ && M <= 1344)))
-    return M <= 512 ? MM_WR_T : MM_WR_S;
-  // gate_up and down of short calls: register-weight blocks too (FDLLM_WR_FFN picks 64 x 128 or 128 x 128 blocks
-  // below 1024 rows, or the LDS-staged kernels).
-  if (M >= 33 && M < 1024 && pol.wr_ffn >= 0 && (cfg == CFG_GATE_UP || cfg == CFG_DOWN)) {
-    const int sh = cfg == CFG_GATE_UP ? 0 : 1;
-    if ((pol.wr_ffn >> sh) & 1) return MM_WR_S;
-    if ((pol.wr_ffn >> (sh + 2)) & 1) return MM_WR_M;
-  } else if (M >= 33 && cfg == CFG_GATE_UP) {
-    // us per launch including its norm pass, k groups / 64 x 128 / 128 x 128 / LDS-staged blocks: 33 rows 17.5 /
-    // 20.5, 64 rows 18.5 / 21.0 / 22.7, 96 rows 20.5 / - / 24.1, 128 rows 23.3 / 29.9 / 26.0, 129 rows 30.8 / 27.2 /
-    // 31.6, 192 rows 32.5 / 28.8 / 34.2, 208 rows - / 34.5 / 35.0, 256 rows 37.6 / 37.5 / 37.1 / 43.2, 320 rows - / 37.8
-    // / 34.9 / 41.7, 384 rows - / 43.2 / 36.6 / 42.1, 416 rows - / 44.3 / 43.0 / 42.0, 512 rows - / 54.1 / 48.8 / 42.6
-    if (M <= 128 && ntiles % WkGu8::bn_tiles == 0) return M <= 64 ? MM_WK_GU4 : M <= 96 ? MM_WK_GU6 : MM_WK_GU8;
-    if (M <= 224) return MM_WR_S;
-    if (M <= 400) return MM_WR_M;
-  } else if (M >= 33 && cfg == CFG_DOWN) {
-    // us per launch with its split sum, 64 x 128 blocks / LDS-staged: 64 rows 14.4 / 21.4, 128 rows 15.7 / 21.4, 192
-    // rows 16.7 / 27.1, 256 rows 17.8 / 22.6, 320 rows 20.9 / 23.8, 352 rows 27.7 / 24.1.  From 417 to 672 rows
-    // 128 x 128 blocks: in a prefill, us per layer against the LDS-staged blocks: 448 rows 90.7 / 93.0, 509 rows
-    // 91.6 / 93.5, 576 rows 102.4 / 109.3, 640 rows 104.9 / 111.3 (but 384 rows 95.4 / 88.5, 768 rows 126.3 / 120.6)
-    if (M <= 320) return MM_WR_S;
-    if (M > 416 && M <= 672) return MM_WR_M;
-  }
-  switch (cfg) {
-    case CFG_LM_HEAD: return MM_WIDE;  // one 256-column confidence tile per block column
-    case CFG_GATE_UP:
-      if (M > 256 && M <= pol.wt256 && ntiles % WtB256::bn_tiles == 0) return MM_WT_256;
-      if (M >= 256 && ntiles % WtBig::bn_tiles == 0) return (pol.wt8 & 1) ? MM_WT_8 : MM_WT;
-      return M >= 1024 ? MM_BIG : MM_WIDE;
-    case CFG_DOWN:
-      if (M >= 256 && ntiles % WtBig::bn_tiles == 0) return (pol.wt8 & 2) ? MM_WT_8 : MM_WT;
-      return M >= 1024 ? MM_WIDE_D : MM_SMALL;
-    default:  // qkv, o_proj: the LDS-staged kernel measured slower at their widths (2048 / 1536 columns)
-      return MM_SMALL;
-  }
-}
+static_assert(mm_is<MmSmall>(MM_SMALL) && mm_is<MmWide>(MM_WIDE) && mm_is<MmWideD>(MM_WIDE_D) && mm_is<MmBig>(MM_BIG) &&
+              mm_is<WtBig>(MM_WT) && mm_is<WtBig8>(MM_WT_8) && mm_is<WtB256>(MM_WT_256) && mm_is<WrBig>(MM_WR) &&
+              mm_is<WrSmall>(MM_WR_S) && mm_is<WrMid>(MM_WR_M) && mm_is<WrTiny>(MM_WR_T) && mm_is<WrB3>(MM_WR_3) &&
+              mm_is<WkGu4>(MM_WK_GU4) && mm_is<WkGu6>(MM_WK_GU6) && mm_is<WkGu8>(MM_WK_GU8), "block sizes");
 
 GemmPlan gemm_plan(int cfg, GemmP& a, int stream_split, const MmPolicy& pol) {
   GemmPlan p{};
@@ -322,45 +231,7 @@ GemmPlan gemm_plan(int cfg, GemmP& a, int stream_split, const MmPolicy& pol) {
       p.mm_id = id;
       p.nbm = (a.M + mi.bm - 1) / mi.bm;
       p.nbn = (a.ntiles + mi.bn_tiles - 1) / mi.bn_tiles;
-      // k split: the smallest divisor of the stage count that brings the launch to mm_target_wgs
-      // workgroups (at most 8 splits of at least mm_min_stages stages), else the largest such divisor
-      const int wgs = p.nbm * p.nbn;
-      // (up to 128 rows, half the target: a split's fp32 partials and its epilogue launch cost more
-      // than the idle compute units; measured on the 128-row batched step, 3.15 -> 2.93 ms)
-      // o_proj (48 k steps) a quarter: at 512 rows its 96 workgroups without a split took 15.4 us against
-      // 18.9 us split three ways with the epilogue launch
-      int target = a.M <= 128 ? pol.target_wgs / 2 : pol.target_wgs;
-      if (cfg == CFG_OPROJ) target /= 4;
-      // qkv on the 64 x 128 (and 64 x 64) register-weight blocks half: 17.1 against 20.4 us at 512 rows (128 workgroups
-      // without a split against 256 with one), 13.8 against 14.5 at 128 (two splits against four)
-      if (cfg == CFG_QKV && (id == MM_WR_S || id == MM_WR_T)) target /= 2;
-      // down above 128 rows seven eighths: at 512 rows seven splits (224 workgroups) against eight (256)
-      // measured 3.92 against 3.94-3.95 ms per batched step (fewer partials for the split sum; five
-      // splits 4.03, ten 3.95)
-      if (cfg == CFG_DOWN && a.M > 128) target = target * 7 / 8;
-      if (id == MM_WT_256 || (id >= MM_WK_GU4 && id <= MM_WK_GU8)) target = 0;  // no split
-      int split = 1;
-      const int max_split = id == MM_WR || id == MM_WR_S || id == MM_WR_M || id == MM_WR_T || id == MM_WR_3 ? 16 : 8;
-      if (pol.force_split > 1 && cfg != CFG_LM_HEAD && nst % pol.force_split == 0 && nst / pol.force_split >= pol.min_stages)
-        split = pol.force_split;
-      else
-        for (int d = 2; d <= max_split && wgs * split < target && cfg != CFG_LM_HEAD; ++d)
-          if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
-      if (cfg == CFG_DOWN && id == MM_WR && pol.wr_min_rows == 0 && pol.force_split <= 1 && pol.target_wgs >= 256) {
-        // (one round: at 1152 rows five splits of 54 blocks took 58.9 us, at 1200 four of 60 blocks 47.8)
-        split = 1;
-        for (int d = 2; d <= max_split && wgs * d <= pol.target_wgs; ++d)
-          if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
-      }
-      if (cfg == CFG_DOWN && id == MM_WR_S && pol.wr_ffn < 0 && pol.force_split <= 1 && pol.target_wgs >= 256) {
-        // down's 64 x 128 blocks: the most splits up to seven that leave every XCD a workgroup per compute unit
-        // at most (us per launch with its split sum; 130 rows: 5 splits 16.7, 7 splits 21.5, of 35 workgroups on
-        // seven XCDs; 64 rows: 7 splits 14.4, 14 splits 16.8, whose partials cost more than their workgroups give)
-        const int fit = std::min(7, std::max(1, pol.target_wgs / 8 / ((wgs + 7) / 8)));
-        split = 1;
-        for (int d = 2; d <= fit; ++d)
-          if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
-      }
+      const int split = mm_split(cfg, id, a.M, a.ntiles, nst, pol);
       p.ksplit = split;
       a.kps = a.KS / split;
       p.part_floats = split > 1 ? (size_t)split * a.ntiles * ((a.M + 15) / 16) * 256 : 0;

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "mm_choice.hpp"
+
 namespace fdllm {
 
 // ---- packed weights ----------------------------------------------------------------------------
@@ -91,8 +93,7 @@ struct GemmP {
   RopeOut ro;                         // EPI_BIAS (qkv) on the register-weight kernel: ro.rope set, see RopeOut
 };
 
-// Launch configurations (see gemm.hip); the host picks one per projection.
-enum GemmCfg : int { CFG_QKV = 0, CFG_OPROJ = 1, CFG_GATE_UP = 2, CFG_DOWN = 3, CFG_LM_HEAD = 4 };
+// Launch configurations (GemmCfg; see gemm.hip): the host picks one per projection.
 // tiles_per_wg: the padding unit of the packed tile count (every kernel of the projection divides it)
 struct GemmShape { int tiles_per_wg; int waves; };
 GemmShape gemm_shape(int cfg);
@@ -109,31 +110,6 @@ struct GemmPlan {
   int mm_id; int nbm; int nbn;
   int tail_full, tail_split;  // GK_STREAM: see GemmP (set in both)
   int mrows;                  // GK_ONESHOT: rows per m-chunk (blockIdx.z), 32, or 16 for half-row chunks
-};
-// How large-M launches are planned.  target_wgs / min_stages: k is split only while the launch has fewer
-// than target_wgs workgroups, and only into splits of at least min_stages stages.  wr_ops: the
-// projections (bit cfg) that may take the register-weight kernel's large blocks, from wr_min_rows rows (0: the
-// row counts where they measured faster than the LDS-staged and streaming kernels, mm_choice).
-struct MmPolicy {
-  int target_wgs = 256;
-  int min_stages = 8;
-  int wr_ops = (1 << CFG_QKV) | (1 << CFG_OPROJ) | (1 << CFG_GATE_UP) | (1 << CFG_DOWN) | (1 << CFG_LM_HEAD);
-  int wr_min_rows = 0;
-  int wr_small_ops = (1 << CFG_QKV) | (1 << CFG_OPROJ);  // take the 64 x 128 register-weight blocks below the 128 x 256 ones
-  // gate_up / down below 1024 rows: -1 the measured choice, else bit 0 / 1 the 64 x 128 register-weight blocks,
-  // bit 2 / 3 the 128 x 128 ones (0: the LDS-staged kernels)
-  int wr_ffn = -1;
-  int force_split = 0;  // > 1: this k split whenever it divides the stages (the fused o_proj + norm)
-  int wr3 = 1;          // o_proj / down at the register-weight thresholds: 128 x 192 blocks (0: 128 x 256)
-  int wt8 = 1;  // LDS-staged 128 x 192 blocks of eight waves (bit 0 gate_up, bit 1 down) instead of four
-  int wt256 = 512;  // gate_up from 257 up to this many rows on LDS-staged 256 x 192 blocks of eight waves
-  // the streaming lm_head of up to 32 rows: the column groups past the last whole round over this many
-  // compute units (one group per unit per round) split k up to 3 ways, so that every unit streams about
-  // the same bytes (0: off)
-  int lm_tail_cus = 0;
-  // one-shot projections (bit cfg) of 17 to 32 rows run as two 16-row m-chunks: each workgroup takes in
-  // half the activations for the same weight tile
-  int os_half = (1 << CFG_QKV) | (1 << CFG_OPROJ);
 };
 GemmPlan gemm_plan(int cfg, GemmP& a, int stream_split, const MmPolicy& pol = MmPolicy{});
 // whether the plan runs the one-shot register-fragment body, the only one that takes xfrag / yfrag 1

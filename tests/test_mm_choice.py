@@ -1,0 +1,54 @@
+"""Which blocks and k splits the large-M projections take (csrc/mm_choice.hpp), on the CPU: the header is host code,
+compiled with g++ and run for given widths."""
+
+from __future__ import annotations
+
+import pathlib
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = pathlib.Path(__file__).resolve().parents[1]
+OPROJ, GATE_UP, DOWN = 1, 2, 3
+# MmId
+LDS_64x128, LDS_64x256, LDS_128x256, LDS_128x192, WR_128x256, WR_64x128, WR_128x128, WR_64x64, WR_128x192 = 0, 2, 3, 4, 5, 6, 7, 8, 9
+LDS_128x192_8W, LDS_256x192, WK_64, WK_96, WK_128 = 10, 11, 12, 13, 14
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ is not available")
+
+
+@pytest.fixture(scope="module")
+def runs(tmp_path_factory):
+    """runs(cfg, rows of the weight, its columns): [(first row count, last, kernel, k splits), ...] of 33 to 8192."""
+    exe = tmp_path_factory.mktemp("mm") / "mm_choice_check"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I", str(ROOT / "fast-dllm-relax_amd" / "csrc"),
+                    str(ROOT / "tests" / "mm_choice_check.cpp"), "-o", str(exe)], check=True)
+
+    def get(cfg, n, k, cus=256):
+        tiles = -(-n // 16 // 12) * 12 if cfg == GATE_UP else n // 16  # (packed in whole workgroups of 12 tiles)
+        out = subprocess.run([str(exe), str(cfg), str(tiles), str(k // 32), str(cus)], capture_output=True, text=True, check=True)
+        return [tuple(int(x) for x in line.split()) for line in out.stdout.splitlines()]
+
+    return get
+
+
+def at(table, rows):
+    return next((kernel, splits) for first, last, kernel, splits in table if first <= rows <= last)
+
+
+def test_1p5b_choices(runs):
+    """The choices at the 1.5B widths, whose times stand beside them in mm_choice.hpp."""
+    assert runs(OPROJ, 1536, 1536) == [
+        (33, 64, WR_64x64, 2), (65, 512, WR_64x64, 1), (513, 1344, WR_64x128, 1), (1345, 2560, LDS_64x128, 1),
+        (2561, 8192, WR_128x192, 1)]
+    assert runs(GATE_UP, 17920, 1536) == [
+        (33, 64, WK_64, 1), (65, 96, WK_96, 1), (97, 128, WK_128, 1), (129, 224, WR_64x128, 1), (225, 400, WR_128x128, 1),
+        (401, 512, LDS_256x192, 1), (513, 640, LDS_128x192_8W, 1), (641, 896, WR_128x256, 1), (897, 2047, LDS_128x192_8W, 1),
+        (2048, 8192, WR_128x256, 1)]
+    assert runs(DOWN, 1536, 8960) == [
+        (33, 128, WR_64x128, 7), (129, 256, WR_64x128, 5), (257, 320, WR_64x128, 4), (321, 384, LDS_128x192, 8),
+        (385, 416, LDS_128x192, 7), (417, 512, WR_128x128, 5), (513, 672, WR_128x128, 4), (673, 768, WR_128x192, 5),
+        (769, 1024, WR_128x192, 4), (1025, 1280, WR_128x256, 4), (1281, 1536, LDS_128x192, 4), (1537, 1664, WR_128x192, 4),
+        (1665, 2048, WR_128x192, 2), (2049, 2560, WR_128x256, 2), (2561, 3200, LDS_128x192, 2), (3201, 3456, WR_128x192, 2),
+        (3457, 8192, WR_128x192, 1)]
