@@ -746,7 +746,7 @@ int fdllm_create(const fdllm_config* cfg, fdllm_ctx** out) {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->dev) == hipSuccess && cus > 0) c->ncu = cus;
     else (void)hipGetLastError();
-    c->mm.lm_tail_cus = c->ncu;
+    c->mm.cus = c->mm.lm_tail_cus = c->ncu;
     if (const char* e = std::getenv("FDLLM_LM_TAIL")) c->mm.lm_tail_cus = atoi(e) != 0 ? c->ncu : 0;
   }
   {

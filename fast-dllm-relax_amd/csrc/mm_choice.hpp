@@ -13,6 +13,7 @@ enum GemmCfg : int { CFG_QKV = 0, CFG_OPROJ = 1, CFG_GATE_UP = 2, CFG_DOWN = 3, 
 // projections (bit cfg) that may take the register-weight kernel's large blocks, from wr_min_rows rows (0: the
 // row counts where they measured faster than the LDS-staged and streaming kernels, mm_choice).
 struct MmPolicy {
+  int cus = 256;  // compute units
   int target_wgs = 256;
   int min_stages = 8;
   int wr_ops = (1 << CFG_QKV) | (1 << CFG_OPROJ) | (1 << CFG_GATE_UP) | (1 << CFG_DOWN) | (1 << CFG_LM_HEAD);
@@ -82,17 +83,21 @@ inline int mm_blocks(int id, int M, int ntiles) {
   const MmInfo b = mm_info(id);
   return (M + b.bm - 1) / b.bm * ((ntiles + b.bn_tiles - 1) / b.bn_tiles);
 }
+// Whether wgs workgroups leave at most 7 of every 32 units of a round of `units` idle.  (gate_up of 896 x 4864: 390
+// blocks of 128 x 256 for two workgroups per unit, 512, take 34.3 us against the LDS-staged 29.8 at 1200 rows, 429
+// 34.6 against 39.2 at 1344; of 2048 x 5632: 405 62.2 against 71.8 at 1100.)
+inline bool mm_fills(int wgs, int units) { return wgs <= units && 32 * wgs > 25 * units; }
 inline int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
-  // The large blocks by how their counts fill the 256 compute units (two workgroups each), us per launch.
-  // Register-weight 128 x 256 gate_up of 641 to 896 rows, one round of at most 490 blocks / LDS-staged: 50.7 /
-  // 56.7 at 660 rows, 51.7 / 59.4 at 896 (but 51.3 / 43.9 at 640, 68.3 / 59.1 at 900).  o_proj past 2560 rows, where
+  // The large blocks, us per launch at the 1.5B shapes.
+  // gate_up on register-weight 128 x 256 where those are one round of two workgroups per unit (641 to 896 rows) / LDS-
+  // staged: 50.7 / 56.7 at 660 rows, 51.7 / 59.4 at 896 (but 51.3 / 43.9 at 640, 68.3 / 59.1 at 900).  o_proj past 2560 rows, where
   // its 64 x 128 blocks start a second round: register-weight 128 x 192 / 64 x 128: 28.6 / 36.0 at 2700, 28.8 / 36.7
   // at 3000 (28.5 / 23.9 at 2560).  Down, register-weight 128 x 192 / LDS-staged: 31.9 / 33.8 at 680 rows, 37.6 / 40.3
   // at 896, 39.4 / 41.3 at 1024, 55.5 / 52.5 at 1100, 59.9 / 59.4 at 1400, 61.7 / 64.1 at 1600, 101 / 97 at 2800, 98 / 105
   // at 3500; 128 x 256 where their splits come to one round, 47.8 / 53.4 at 1200, 78.6 / 86.9 at 2100, 79.4 / 90.1 at 2400.
   if (pol.wr_min_rows == 0 && ((pol.wr_ops >> cfg) & 1) && pol.wr_ffn < 0) {
     const bool b3 = pol.wr3 && ntiles % 12 == 0;
-    if (cfg == CFG_GATE_UP && M > 640 && M <= 896) return MM_WR;
+    if (cfg == CFG_GATE_UP && M > 400 && mm_fills(mm_blocks(MM_WR, M, ntiles), 2 * pol.cus)) return MM_WR;
     if (cfg == CFG_OPROJ && M > 2560 && b3) return MM_WR_3;
     if (cfg == CFG_DOWN && ((M > 1024 && M <= 1280) || (M > 2048 && M <= 2560))) return MM_WR;
     if (cfg == CFG_DOWN && ((M > 672 && M <= 1024) || (M > 1536 && M <= 2048)) && b3) return MM_WR_3;
@@ -123,7 +128,8 @@ inline int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
     // / 34.9 / 41.7, 384 rows - / 43.2 / 36.6 / 42.1, 416 rows - / 44.3 / 43.0 / 42.0, 512 rows - / 54.1 / 48.8 / 42.6
     if (M <= 128 && ntiles % 6 == 0) return M <= 64 ? MM_WK_GU4 : M <= 96 ? MM_WK_GU6 : MM_WK_GU8;
     if (M <= 224) return MM_WR_S;
-    if (M <= 400) return MM_WR_M;
+    // (2048 x 11008, 519 blocks of 128 x 128 for two workgroups per unit: 53.7 / 51.7 LDS-staged at 300 rows)
+    if (M <= 400 && mm_blocks(MM_WR_M, M, ntiles) <= 2 * pol.cus) return MM_WR_M;
   } else if (M >= 33 && cfg == CFG_DOWN) {
     // us per launch with its split sum, 64 x 128 blocks / LDS-staged: 64 rows 14.4 / 21.4, 128 rows 15.7 / 21.4, 192
     // rows 16.7 / 27.1, 256 rows 17.8 / 22.6, 320 rows 20.9 / 23.8, 352 rows 27.7 / 24.1.  From 417 to 672 rows

@@ -11,7 +11,7 @@ int main(int argc, char** argv) {
   if (argc != 5) return 1;
   const int cfg = atoi(argv[1]), ntiles = atoi(argv[2]), ks = atoi(argv[3]);
   MmPolicy pol;
-  (void)argv[4];
+  pol.cus = atoi(argv[4]);
   int first = 33, id0 = -1, split0 = 0;
   for (int M = 33; M <= 8193; ++M) {
     int id = -1, split = 0;

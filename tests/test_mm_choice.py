@@ -43,8 +43,8 @@ def test_1p5b_choices(runs):
         (33, 64, WR_64x64, 2), (65, 512, WR_64x64, 1), (513, 1344, WR_64x128, 1), (1345, 2560, LDS_64x128, 1),
         (2561, 8192, WR_128x192, 1)]
     assert runs(GATE_UP, 17920, 1536) == [
-        (33, 64, WK_64, 1), (65, 96, WK_96, 1), (97, 128, WK_128, 1), (129, 224, WR_64x128, 1), (225, 400, WR_128x128, 1),
-        (401, 512, LDS_256x192, 1), (513, 640, LDS_128x192_8W, 1), (641, 896, WR_128x256, 1), (897, 2047, LDS_128x192_8W, 1),
+        (33, 64, WK_64, 1), (65, 96, WK_96, 1), (97, 128, WK_128, 1), (129, 224, WR_64x128, 1), (225, 384, WR_128x128, 1),
+        (385, 512, LDS_256x192, 1), (513, 640, LDS_128x192_8W, 1), (641, 896, WR_128x256, 1), (897, 2047, LDS_128x192_8W, 1),
         (2048, 8192, WR_128x256, 1)]
     assert runs(DOWN, 1536, 8960) == [
         (33, 128, WR_64x128, 7), (129, 256, WR_64x128, 5), (257, 320, WR_64x128, 4), (321, 384, LDS_128x192, 8),
@@ -52,3 +52,17 @@ def test_1p5b_choices(runs):
         (769, 1024, WR_128x192, 4), (1025, 1280, WR_128x256, 4), (1281, 1536, LDS_128x192, 4), (1537, 1664, WR_128x192, 4),
         (1665, 2048, WR_128x192, 2), (2049, 2560, WR_128x256, 2), (2561, 3200, LDS_128x192, 2), (3201, 3456, WR_128x192, 2),
         (3457, 8192, WR_128x192, 1)]
+
+
+def test_gate_up_blocks_follow_their_count(runs):
+    """gate_up takes register-weight 128 x 256 blocks below 2048 rows where they fill one round of two workgroups per
+    compute unit, whatever the width and the device."""
+    for n, k, rows in [(9728, 896, (641, 700, 896, 1200)), (5632, 1024, (641, 800, 896)), (11264, 2048, (641, 700, 800, 896)),
+                       (22016, 2048, (641, 700, 896)), (2304, 640, (641, 700, 896))]:
+        for r in rows:
+            assert at(runs(GATE_UP, n, k), r)[0] == LDS_128x192_8W, (n, k, r)
+    for n, k, rows in [(9728, 896, (1281, 1600)), (11264, 2048, (1100, 1400)), (22016, 2048, (513, 640))]:
+        for r in rows:
+            assert at(runs(GATE_UP, n, k), r)[0] == WR_128x256, (n, k, r)
+    assert at(runs(GATE_UP, 22016, 2048), 300)[0] == LDS_256x192  # 519 blocks of 128 x 128
+    assert at(runs(GATE_UP, 17920, 1536, cus=128), 700)[0] == LDS_128x192_8W
