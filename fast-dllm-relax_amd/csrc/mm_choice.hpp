@@ -90,15 +90,15 @@ inline bool mm_fills(int wgs, int units) { return wgs <= units && 32 * wgs > 25 
 inline int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
   // The large blocks, us per launch at the 1.5B shapes.
   // gate_up on register-weight 128 x 256 where those are one round of two workgroups per unit (641 to 896 rows) / LDS-
-  // staged: 50.7 / 56.7 at 660 rows, 51.7 / 59.4 at 896 (but 51.3 / 43.9 at 640, 68.3 / 59.1 at 900).  o_proj past 2560 rows, where
-  // its 64 x 128 blocks start a second round: register-weight 128 x 192 / 64 x 128: 28.6 / 36.0 at 2700, 28.8 / 36.7
-  // at 3000 (28.5 / 23.9 at 2560).  Down, register-weight 128 x 192 / LDS-staged: 31.9 / 33.8 at 680 rows, 37.6 / 40.3
+  // staged: 50.7 / 56.7 at 660 rows, 51.7 / 59.4 at 896 (but 51.3 / 43.9 at 640, 68.3 / 59.1 at 900).  o_proj on
+  // register-weight 128 x 192 once its 64 x 128 blocks pass two workgroups per unit (2688 rows) / 64 x 128: 28.6 / 36.0
+  // at 2700, 28.8 / 36.7 at 3000 (28.9 / 24.1 at 2688).  Down, register-weight 128 x 192 / LDS-staged: 31.9 / 33.8 at 680 rows, 37.6 / 40.3
   // at 896, 39.4 / 41.3 at 1024, 55.5 / 52.5 at 1100, 59.9 / 59.4 at 1400, 61.7 / 64.1 at 1600, 101 / 97 at 2800, 98 / 105
   // at 3500; 128 x 256 where their splits come to one round, 47.8 / 53.4 at 1200, 78.6 / 86.9 at 2100, 79.4 / 90.1 at 2400.
   if (pol.wr_min_rows == 0 && ((pol.wr_ops >> cfg) & 1) && pol.wr_ffn < 0) {
     const bool b3 = pol.wr3 && ntiles % 12 == 0;
     if (cfg == CFG_GATE_UP && M > 400 && mm_fills(mm_blocks(MM_WR, M, ntiles), 2 * pol.cus)) return MM_WR;
-    if (cfg == CFG_OPROJ && M > 2560 && b3) return MM_WR_3;
+    if (cfg == CFG_OPROJ && b3 && mm_blocks(MM_SMALL, M, ntiles) > 2 * pol.cus) return MM_WR_3;
     if (cfg == CFG_DOWN && ((M > 1024 && M <= 1280) || (M > 2048 && M <= 2560))) return MM_WR;
     if (cfg == CFG_DOWN && ((M > 672 && M <= 1024) || (M > 1536 && M <= 2048)) && b3) return MM_WR_3;
     if (cfg == CFG_DOWN && M > 2560 && M <= 3200 && ntiles % 12 == 0) return MM_WT;
@@ -112,8 +112,9 @@ inline int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
   // 23.3 / 26.4 at 2048 (equal below 384).  Up to 512 rows 64 x 64 blocks, twice the workgroups, do better
   // still (us, 64 x 128 / 64 x 64 blocks): qkv 14.4 / 13.4 at 128 rows, 15.7 / 13.7 at 256, 16.8 / 14.9 at
   // 512 (but 19.4 / 21.2 at 1024); o_proj 12.8 / 11.9, 12.8 / 11.9, 14.0 / 12.0 (15.1 / 21.4 at 1024)
-  // o_proj up to 1344 rows, one round of 64 x 128 blocks (16.1 / 20.0 at 1300 rows, 25.9 / 23.3 at 1500)
-  if (M >= 33 && ((pol.wr_small_ops >> cfg) & 1) && (cfg == CFG_QKV || (cfg == CFG_OPROJ && M <= 1344)))
+  // o_proj while its 64 x 128 blocks are one round of the compute units (1344 rows: 16.1 / 20.0 at 1300, 25.9 / 23.3
+  // at 1500; 896 columns, 2304 rows: 17.0 / 22.7 at 1800, 17.4 / 23.0 at 2300)
+  if (M >= 33 && ((pol.wr_small_ops >> cfg) & 1) && (cfg == CFG_QKV || (cfg == CFG_OPROJ && mm_blocks(MM_WR_S, M, ntiles) <= pol.cus)))
     return M <= 512 ? MM_WR_T : MM_WR_S;
   // gate_up and down of short calls: register-weight blocks too (FDLLM_WR_FFN picks 64 x 128 or 128 x 128 blocks
   // below 1024 rows, or the LDS-staged kernels).

@@ -40,8 +40,8 @@ def at(table, rows):
 def test_1p5b_choices(runs):
     """The choices at the 1.5B widths, whose times stand beside them in mm_choice.hpp."""
     assert runs(OPROJ, 1536, 1536) == [
-        (33, 64, WR_64x64, 2), (65, 512, WR_64x64, 1), (513, 1344, WR_64x128, 1), (1345, 2560, LDS_64x128, 1),
-        (2561, 8192, WR_128x192, 1)]
+        (33, 64, WR_64x64, 2), (65, 512, WR_64x64, 1), (513, 1344, WR_64x128, 1), (1345, 2688, LDS_64x128, 1),
+        (2689, 8192, WR_128x192, 1)]
     assert runs(GATE_UP, 17920, 1536) == [
         (33, 64, WK_64, 1), (65, 96, WK_96, 1), (97, 128, WK_128, 1), (129, 224, WR_64x128, 1), (225, 384, WR_128x128, 1),
         (385, 512, LDS_256x192, 1), (513, 640, LDS_128x192_8W, 1), (641, 896, WR_128x256, 1), (897, 2047, LDS_128x192_8W, 1),
@@ -66,3 +66,11 @@ def test_gate_up_blocks_follow_their_count(runs):
             assert at(runs(GATE_UP, n, k), r)[0] == WR_128x256, (n, k, r)
     assert at(runs(GATE_UP, 22016, 2048), 300)[0] == LDS_256x192  # 519 blocks of 128 x 128
     assert at(runs(GATE_UP, 17920, 1536, cus=128), 700)[0] == LDS_128x192_8W
+
+
+def test_o_proj_blocks_follow_their_count(runs):
+    """o_proj keeps the register-weight 64 x 128 blocks while they are one round, at any width, and leaves the LDS-
+    staged ones only when those pass two workgroups per compute unit."""
+    for n, last in [(640, 3264), (896, 2304), (1024, 2048), (1536, 1344), (2048, 1024)]:
+        table = runs(OPROJ, n, n)
+        assert at(table, last)[0] == WR_64x128 and at(table, last + 1)[0] == LDS_64x128, n
