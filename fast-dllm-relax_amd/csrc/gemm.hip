@@ -223,7 +223,7 @@ GemmPlan gemm_plan(int cfg, GemmP& a, int stream_split, const MmPolicy& pol) {
   GemmPlan p{};
   p.mchunks = (a.M + 31) / 32;
   if (a.M > 32) {
-    const int id = mm_choice(cfg, a.M, a.ntiles, pol);
+    const int id = mm_choice(cfg, a.M, a.ntiles, a.KS, pol);
     const MmInfo mi = mm_info(id);
     if (a.KS % mi.kss == 0) {
       const int nst = a.KS / mi.kss;

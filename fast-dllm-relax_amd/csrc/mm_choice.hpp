@@ -83,25 +83,46 @@ inline int mm_blocks(int id, int M, int ntiles) {
   const MmInfo b = mm_info(id);
   return (M + b.bm - 1) / b.bm * ((ntiles + b.bn_tiles - 1) / b.bn_tiles);
 }
-// Whether wgs workgroups leave at most 7 of every 32 units of a round of `units` idle.  (gate_up of 896 x 4864: 390
-// blocks of 128 x 256 for two workgroups per unit, 512, take 34.3 us against the LDS-staged 29.8 at 1200 rows, 429
-// 34.6 against 39.2 at 1344; of 2048 x 5632: 405 62.2 against 71.8 at 1100.)
+// Whether wgs workgroups leave at most 7 of every 32 units of a round of `units` idle.  (The line lies between down of
+// 3100 rows, 200 blocks of 128 x 192 on 256 units, 102.7 us against the LDS-staged 99.5, and of 2200 rows, 204 of
+// 128 x 256, 77.3 against 92.3; gate_up of 896 x 4864, 390 blocks of 128 x 256 for 512, 34.3 against 29.8 at 1200 rows,
+// 429 for 512, 34.6 against 39.2 at 1344.)
 inline bool mm_fills(int wgs, int units) { return wgs <= units && 32 * wgs > 25 * units; }
-inline int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
-  // The large blocks, us per launch at the 1.5B shapes.
+// The most k splits, of at least 16 stages each, of nb blocks within one round of a workgroup per compute unit (0: the
+// blocks alone are more).
+inline int mm_round_split(int nb, int nst, const MmPolicy& pol) {
+  int split = nb <= pol.cus ? 1 : 0;
+  for (int d = 2; d <= 16 && nb * d <= pol.cus; ++d)
+    if (nst % d == 0 && nst / d >= std::max(16, pol.min_stages)) split = d;
+  return split;
+}
+// Down on register-weight 128 x 256 blocks whose splits come to one round: where they fill it, or, for weights
+// that are no whole number of 192-column blocks (the LDS-staged 64 x 256 blocks take those below 2048 rows), take
+// more than half of it (2048 x 5632, us: 53 against 67 at 1100 rows, 56 / 72 at 1700; 896 x 4864: 29 / 36, 32 / 40).
+inline bool mm_down_round(int M, int ntiles, int ks, const MmPolicy& pol) {
+  const int nb = mm_blocks(MM_WR, M, ntiles), wgs = nb * mm_round_split(nb, ks, pol);
+  if (ntiles % 12 == 0) return mm_blocks(MM_WR_3, M, ntiles) <= pol.cus && mm_fills(wgs, pol.cus);
+  return M < 2048 && 2 * wgs > pol.cus;
+}
+inline int mm_choice(int cfg, int M, int ntiles, int ks, const MmPolicy& pol) {
+  // The large blocks by how their counts fill the compute units, us per launch at the 1.5B shapes.
   // gate_up on register-weight 128 x 256 where those are one round of two workgroups per unit (641 to 896 rows) / LDS-
   // staged: 50.7 / 56.7 at 660 rows, 51.7 / 59.4 at 896 (but 51.3 / 43.9 at 640, 68.3 / 59.1 at 900).  o_proj on
   // register-weight 128 x 192 once its 64 x 128 blocks pass two workgroups per unit (2688 rows) / 64 x 128: 28.6 / 36.0
-  // at 2700, 28.8 / 36.7 at 3000 (28.9 / 24.1 at 2688).  Down, register-weight 128 x 192 / LDS-staged: 31.9 / 33.8 at 680 rows, 37.6 / 40.3
-  // at 896, 39.4 / 41.3 at 1024, 55.5 / 52.5 at 1100, 59.9 / 59.4 at 1400, 61.7 / 64.1 at 1600, 101 / 97 at 2800, 98 / 105
-  // at 3500; 128 x 256 where their splits come to one round, 47.8 / 53.4 at 1200, 78.6 / 86.9 at 2100, 79.4 / 90.1 at 2400.
+  // at 2700, 28.8 / 36.7 at 3000 (28.9 / 24.1 at 2688).  Down, register-weight 128 x 192 where those fill a round /
+  // LDS-staged: 31.6 / 33.1 at 660 rows (128 x 128 blocks, one and an eighth rounds: 42.2), 37.6 / 40.3 at 896, 39.4 / 41.3
+  // at 1024, 55.5 / 52.5 at 1100, 59.9 / 59.4 at 1400, 61.7 / 64.1 at 1600, 101 / 97 at 2800, 98 / 105 at 3500; 128 x 256
+  // where those do, 47.8 / 53.4 at 1200, 78.6 / 86.9 at 2100, 79.4 / 90.1 at 2400, 82.4 / 95.6 at 2688.
   if (pol.wr_min_rows == 0 && ((pol.wr_ops >> cfg) & 1) && pol.wr_ffn < 0) {
     const bool b3 = pol.wr3 && ntiles % 12 == 0;
     if (cfg == CFG_GATE_UP && M > 400 && mm_fills(mm_blocks(MM_WR, M, ntiles), 2 * pol.cus)) return MM_WR;
     if (cfg == CFG_OPROJ && b3 && mm_blocks(MM_SMALL, M, ntiles) > 2 * pol.cus) return MM_WR_3;
-    if (cfg == CFG_DOWN && ((M > 1024 && M <= 1280) || (M > 2048 && M <= 2560))) return MM_WR;
-    if (cfg == CFG_DOWN && ((M > 672 && M <= 1024) || (M > 1536 && M <= 2048)) && b3) return MM_WR_3;
-    if (cfg == CFG_DOWN && M > 2560 && M <= 3200 && ntiles % 12 == 0) return MM_WT;
+    if (cfg == CFG_DOWN && M > 640) {
+      const int nb = mm_blocks(MM_WR_3, M, ntiles);
+      if (b3 && mm_fills(nb * mm_round_split(nb, ks, pol), pol.cus)) return MM_WR_3;
+      if (mm_down_round(M, ntiles, ks, pol)) return MM_WR;
+      if (ntiles % 12 == 0 && M > 2048 && nb <= pol.cus) return MM_WT;
+    }
   }
   const int min_rows = pol.wr_min_rows > 0 ? pol.wr_min_rows : wr_default_min_rows(cfg);
   if (M >= std::max(min_rows, 33) && ((pol.wr_ops >> cfg) & 1))
@@ -133,11 +154,15 @@ inline int mm_choice(int cfg, int M, int ntiles, const MmPolicy& pol) {
     if (M <= 400 && mm_blocks(MM_WR_M, M, ntiles) <= 2 * pol.cus) return MM_WR_M;
   } else if (M >= 33 && cfg == CFG_DOWN) {
     // us per launch with its split sum, 64 x 128 blocks / LDS-staged: 64 rows 14.4 / 21.4, 128 rows 15.7 / 21.4, 192
-    // rows 16.7 / 27.1, 256 rows 17.8 / 22.6, 320 rows 20.9 / 23.8, 352 rows 27.7 / 24.1.  From 417 to 672 rows
-    // 128 x 128 blocks: in a prefill, us per layer against the LDS-staged blocks: 448 rows 90.7 / 93.0, 509 rows
-    // 91.6 / 93.5, 576 rows 102.4 / 109.3, 640 rows 104.9 / 111.3 (but 384 rows 95.4 / 88.5, 768 rows 126.3 / 120.6)
+    // rows 16.7 / 27.1, 256 rows 17.8 / 22.6, 320 rows 20.9 / 23.8, 352 rows 27.7 / 24.1.  From 417 to 640 rows
+    // 128 x 128 blocks where their splits fill a round (or half of it, as in mm_down_round): in a prefill, us per layer
+    // against the LDS-staged blocks: 448 rows 90.7 / 93.0, 509 rows 91.6 / 93.5, 576 rows 102.4 / 109.3, 640 rows 104.9 /
+    // 111.3 (but 384 rows 95.4 / 88.5, 768 rows 126.3 / 120.6)
     if (M <= 320) return MM_WR_S;
-    if (M > 416 && M <= 672) return MM_WR_M;
+    if (M > 416 && M <= 640) {
+      const int nb = mm_blocks(MM_WR_M, M, ntiles), wgs = nb * mm_round_split(nb, ks, pol);
+      if (ntiles % 12 == 0 ? mm_fills(wgs, pol.cus) : 2 * wgs > pol.cus) return MM_WR_M;
+    }
   }
   switch (cfg) {
     case CFG_LM_HEAD: return MM_WIDE;  // one 256-column confidence tile per block column
@@ -179,12 +204,10 @@ inline int mm_split(int cfg, int id, int M, int ntiles, int nst, const MmPolicy&
   else
     for (int d = 2; d <= max_split && wgs * split < target && cfg != CFG_LM_HEAD; ++d)
       if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
-  if (cfg == CFG_DOWN && id == MM_WR && pol.wr_min_rows == 0 && pol.force_split <= 1 && pol.target_wgs >= 256) {
-    // (one round: at 1152 rows five splits of 54 blocks took 58.9 us, at 1200 four of 60 blocks 47.8)
-    split = 1;
-    for (int d = 2; d <= max_split && wgs * d <= pol.target_wgs; ++d)
-      if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
-  }
+  // (at 1152 rows five splits of 54 blocks took 58.9 us, at 1200 four of 60 blocks 47.8)
+  if (cfg == CFG_DOWN && id == MM_WR && pol.wr_min_rows == 0 && pol.force_split <= 1 && pol.target_wgs >= pol.cus &&
+      mm_down_round(M, ntiles, nst, pol))
+    split = mm_round_split(wgs, nst, pol);
   if (cfg == CFG_DOWN && id == MM_WR_S && pol.wr_ffn < 0 && pol.force_split <= 1 && pol.target_wgs >= 256) {
     // down's 64 x 128 blocks: the most splits up to seven that leave every XCD a workgroup per compute unit
     // at most (us per launch with its split sum; 130 rows: 5 splits 16.7, 7 splits 21.5, of 35 workgroups on

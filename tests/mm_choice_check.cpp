@@ -16,7 +16,7 @@ int main(int argc, char** argv) {
   for (int M = 33; M <= 8193; ++M) {
     int id = -1, split = 0;
     if (M <= 8192) {
-      id = mm_choice(cfg, M, ntiles, pol);
+      id = mm_choice(cfg, M, ntiles, ks, pol);
       const MmInfo b = mm_info(id);
       split = ks % b.kss ? 0 : mm_split(cfg, id, M, ntiles, ks / b.kss, pol);  // 0: the streaming kernel
     }

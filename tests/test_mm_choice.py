@@ -48,9 +48,9 @@ def test_1p5b_choices(runs):
         (2048, 8192, WR_128x256, 1)]
     assert runs(DOWN, 1536, 8960) == [
         (33, 128, WR_64x128, 7), (129, 256, WR_64x128, 5), (257, 320, WR_64x128, 4), (321, 384, LDS_128x192, 8),
-        (385, 416, LDS_128x192, 7), (417, 512, WR_128x128, 5), (513, 672, WR_128x128, 4), (673, 768, WR_128x192, 5),
+        (385, 416, LDS_128x192, 7), (417, 512, WR_128x128, 5), (513, 640, WR_128x128, 4), (641, 768, WR_128x192, 5),
         (769, 1024, WR_128x192, 4), (1025, 1280, WR_128x256, 4), (1281, 1536, LDS_128x192, 4), (1537, 1664, WR_128x192, 4),
-        (1665, 2048, WR_128x192, 2), (2049, 2560, WR_128x256, 2), (2561, 3200, LDS_128x192, 2), (3201, 3456, WR_128x192, 2),
+        (1665, 2048, WR_128x192, 2), (2049, 2688, WR_128x256, 2), (2689, 3200, LDS_128x192, 2), (3201, 3456, WR_128x192, 2),
         (3457, 8192, WR_128x192, 1)]
 
 
@@ -74,3 +74,18 @@ def test_o_proj_blocks_follow_their_count(runs):
     for n, last in [(640, 3264), (896, 2304), (1024, 2048), (1536, 1344), (2048, 1024)]:
         table = runs(OPROJ, n, n)
         assert at(table, last)[0] == WR_64x128 and at(table, last + 1)[0] == LDS_64x128, n
+
+
+def test_down_blocks_follow_their_count(runs):
+    """down's large blocks and their one-round splits where the splits fill the round (or take over half of it against the
+    LDS-staged 64 x 256 blocks), with at least 16 stages each; past that the splits of the other kernels."""
+    # short weights: no round to fill, or only with splits of 9 or 11 stages
+    for r in (450, 660, 1100, 1400):
+        assert at(runs(DOWN, 640, 1152), r)[0] in (LDS_64x128, LDS_64x256), r
+    for r in (450, 660, 800, 1024):
+        assert at(runs(DOWN, 1024, 2816), r)[0] in (LDS_64x128, LDS_64x256), r
+    assert at(runs(DOWN, 1024, 2816), 1100) == (WR_128x256, 4)
+    # from 2048 rows on, widths without 192-column blocks keep the splits that more than one round takes
+    assert at(runs(DOWN, 896, 4864), 2300) == (WR_128x256, 4) and at(runs(DOWN, 2048, 11008), 2300) == (WR_128x256, 2)
+    for n, k in [(896, 4864), (2048, 5632), (2048, 11008)]:
+        assert at(runs(DOWN, n, k), 700)[0] == WR_128x256 and at(runs(DOWN, n, k), 1500)[0] == WR_128x256, (n, k)
