@@ -208,14 +208,19 @@ inline int mm_split(int cfg, int id, int M, int ntiles, int nst, const MmPolicy&
   if (cfg == CFG_DOWN && id == MM_WR && pol.wr_min_rows == 0 && pol.force_split <= 1 && pol.target_wgs >= pol.cus &&
       mm_down_round(M, ntiles, nst, pol))
     split = mm_round_split(wgs, nst, pol);
-  if (cfg == CFG_DOWN && id == MM_WR_S && pol.wr_ffn < 0 && pol.force_split <= 1 && pol.target_wgs >= 256) {
+  if (cfg == CFG_DOWN && id == MM_WR_S && pol.wr_ffn < 0 && pol.force_split <= 1 && pol.target_wgs >= pol.cus) {
     // down's 64 x 128 blocks: the most splits up to seven that leave every XCD a workgroup per compute unit
     // at most (us per launch with its split sum; 130 rows: 5 splits 16.7, 7 splits 21.5, of 35 workgroups on
-    // seven XCDs; 64 rows: 7 splits 14.4, 14 splits 16.8, whose partials cost more than their workgroups give)
-    const int fit = std::min(7, std::max(1, pol.target_wgs / 8 / ((wgs + 7) / 8)));
+    // seven XCDs; 64 rows: 7 splits 14.4, 8 splits 14.7, 14 splits 16.8, whose partials cost more than their workgroups
+    // give).  Eight where none of five to seven divides the stages and four leave over half the units without a
+    // workgroup or more than 64 stages each (four / eight: 2048 x 11008 64 rows 26.8 / 19.5, 128 rows 26.7 / 20.3, 896 x
+    // 4864 40 rows 12.7 / 11.1; but 2048 x 5632 128 rows 14.0 / 14.6).
+    const int fit = std::min(8, std::max(1, pol.target_wgs / 8 / ((wgs + 7) / 8)));
     split = 1;
     for (int d = 2; d <= fit; ++d)
-      if (nst % d == 0 && nst / d >= pol.min_stages) split = d;
+      if (nst % d == 0 && nst / d >= pol.min_stages &&
+          (d < 8 || (split < 5 && (2 * wgs * split < pol.cus || nst / split > 64))))
+        split = d;
   }
   return split;
 }

@@ -89,3 +89,12 @@ def test_down_blocks_follow_their_count(runs):
     assert at(runs(DOWN, 896, 4864), 2300) == (WR_128x256, 4) and at(runs(DOWN, 2048, 11008), 2300) == (WR_128x256, 2)
     for n, k in [(896, 4864), (2048, 5632), (2048, 11008)]:
         assert at(runs(DOWN, n, k), 700)[0] == WR_128x256 and at(runs(DOWN, n, k), 1500)[0] == WR_128x256, (n, k)
+
+
+def test_down_splits_of_short_calls(runs):
+    """down's 64 x 128 blocks take up to seven splits; eight where none of five to seven divides the k stages and four
+    leave units idle or splits long."""
+    for k, rows, splits in [(8960, 64, 7), (11008, 64, 8), (11008, 128, 8), (5632, 64, 8), (5632, 128, 4), (11008, 160, 4)]:
+        n = 1536 if k == 8960 else 2048
+        assert at(runs(DOWN, n, k), rows) == (WR_64x128, splits), (k, rows)
+    assert at(runs(DOWN, 896, 4864), 40) == (WR_64x128, 8)
