@@ -1,5 +1,6 @@
 // Attention launch planning and launchers; the kernels and their bodies are in attn_body.hpp.
 #include "attn_body.hpp"
+#include "prefill_form.hpp"
 
 #include <algorithm>
 
@@ -185,17 +186,8 @@ static hipError_t launch_chunk_mask(const AttnP& a, const AttnPlan& p, hipStream
   }
 }
 
-// Long row blocks: the RoPE + KV append pass (unless qkv's epilogue did it), then attn_prefill_kernel, in one
-// of four forms: all of a kv head's twelve tiles per workgroup (TQ = 3, six query heads per kv head) or four,
-// query blocks paired or alone.  prefill_pair: 0 alone, 2 paired with all tiles, 3 paired with four, 1 by size:
-// four tiles alone until their workgroups pass one round of the 256 compute units by a quarter, then paired
-// (uneven blocks in a second round cost more than the pairs' fewer workgroups), all twelve alone once that
-// gives 180 workgroups and paired once the pairs give 7/8 of a round.  Measured (1.5B bf16
-// build_prefix_cache, us per layer; four alone / four paired / twelve alone / twelve paired): 509 rows 109.8 /
-// 113.7 / 119.2 / 128.2, 1500 rows 226 / 229 / 245 / 254, 2048 rows 271 / 261 / 282 / 291, 3000 rows 386 / 397 /
-// 389 / 398, 4096 rows 494 / 489 / 481 / 487, 6000 rows 762 / 787 / 708 / 716, 8192 rows 1041 / 1025 / 942 / 932.
-constexpr int PREFILL_ALONE_MAX_WGS = 320, PREFILL_WHOLE_MIN_WGS = 180, PREFILL_WHOLE_PAIRED_MIN_WGS = 224;
-
+// Long row blocks: the RoPE + KV append pass (unless qkv's epilogue did it), then attn_prefill_kernel in the form of
+// prefill_form.hpp (TQ = 3: all of a kv head's twelve tiles per workgroup).
 template <int DT, int MASK, int TQ>
 static hipError_t launch_prefill_cfg(const AttnP& a, int paired, hipStream_t st) {
   auto kern = attn_prefill_kernel<DT, MASK, TQ>;
@@ -210,13 +202,8 @@ static hipError_t launch_prefill_cfg(const AttnP& a, int paired, hipStream_t st)
 template <int DT, int MASK>
 static hipError_t launch_prefill(const AttnP& a, hipStream_t st) {
   if (!a.roped) hipLaunchKernelGGL(rope_kv_kernel<DT>, dim3(a.rows), dim3(128), 0, st, a);
-  const int nqb = (a.rows + 31) / 32, grp = a.nq / a.nkv;
-  bool paired = a.prefill_pair >= 2, whole = grp == 6 && (a.prefill_pair == 2 || a.prefill_hpw == 6);
-  if (a.prefill_pair == 1 && !whole && nqb * a.nkv * ((2 * grp + 3) / 4) > PREFILL_ALONE_MAX_WGS) {
-    whole = grp == 6 && nqb * a.nkv >= PREFILL_WHOLE_MIN_WGS;
-    paired = !whole || (nqb + 1) / 2 * a.nkv >= PREFILL_WHOLE_PAIRED_MIN_WGS;
-  }
-  return whole ? launch_prefill_cfg<DT, MASK, 3>(a, paired, st) : launch_prefill_cfg<DT, MASK, 1>(a, paired, st);
+  const PrefillForm f = prefill_form(a.rows, a.nq, a.nkv, a.prefill_pair, a.prefill_hpw);
+  return f.whole ? launch_prefill_cfg<DT, MASK, 3>(a, f.paired, st) : launch_prefill_cfg<DT, MASK, 1>(a, f.paired, st);
 }
 
 // Batched calls without a mask: the RoPE + KV append pass over the call's rows, then attn_seq_kernel.

@@ -98,7 +98,7 @@ struct fdllm_ctx {
   int32_t* zero_i32 = nullptr;
   float* rope = nullptr; size_t rope_floats = 0;  // RoPE (cos, sin) table of the current call's rows
   int attn_target = 64;   // attention workgroups aimed for when splitting the keys
-  int prefill_hpw = 0;    // prefill attention: 6 takes all heads of a kv head per workgroup (AttnP::prefill_hpw)
+  int prefill_hpw = 0;    // prefill attention: query heads per workgroup, 2 or 6 (AttnP::prefill_hpw)
   int prefill_pair = 1;   // prefill attention's query blocks (AttnP::prefill_pair)
   int seq_attn = 1;       // attn_seq_kernel for batched calls and one sequence's longer ones (0: the chunk kernel with
                           // key splits + merge, the loop kernel and the prefill kernel)

@@ -196,9 +196,10 @@ struct AttnP {
   const float* bias; long long bias_ld;
   int S, chunk;                       // key splits (gridDim.z), keys per split (multiple of 32)
   int target_wgs;                     // workgroups the plan aims for (attn_plan)
-  int prefill_hpw;                    // query heads per workgroup of the prefill kernel (6: all of a kv head; else two, or by size)
+  int prefill_hpw;                    // query heads per workgroup of the prefill kernel: 2, 6 (all of a kv head), else by
+                                      // prefill_pair
   int prefill_pair;                   // its query blocks: 0 alone, 1 by size, 2 paired with all heads per workgroup, 3 paired
-                                      // with the heads split over workgroups
+                                      // with the heads split over workgroups (prefill_form.hpp)
   int seq_attn;                       // attn_seq_kernel: a batched call without a mask, or one sequence's (AttnPlan::seq)
   float* part;                        // split partials (merged by attn_merge_kernel)
   uint16_t* out;                      // [rows][nq * 128]

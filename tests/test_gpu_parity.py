@@ -339,8 +339,8 @@ def test_score_masked_continuation_matches_oracle(tiny):
 
 
 def test_prefill_attention_configs_agree(wide2, monkeypatch):
-    """The prefill attention kernel gives every query the same arithmetic whatever the number of query
-    heads per workgroup (1, 2, 3 or 6 of a kv head's 6), so all four give bit-identical outputs."""
+    """The prefill attention kernel gives every query the same arithmetic in each of its four forms (two or all six of
+    a kv head's query heads per workgroup, query blocks alone or paired), so all four give bit-identical outputs."""
     from fast_dllm_relax_amd.config import FastDLLMConfig
     from fast_dllm_relax_amd.params import from_numpy
     from fast_dllm_relax_amd.vm import HipVM
@@ -351,15 +351,16 @@ def test_prefill_attention_configs_agree(wide2, monkeypatch):
     ids = _ids(rng, S, WIDE2["vocab_size"])
     x = vm0.embed(_dev_ids(ids))[None]
     outs = {}
-    for hpw in (1, 2, 3, 6):
+    for pair, hpw in ((0, 2), (0, 6), (2, 0), (3, 0)):
+        monkeypatch.setenv("FDLLM_PREFILL_PAIR", str(pair))
         monkeypatch.setenv("FDLLM_PREFILL_HPW", str(hpw))
         cfg = FastDLLMConfig(**WIDE2)
         vm = HipVM(cfg, from_numpy(ref.p, cfg, dtype="bfloat16"), dtype="bfloat16", max_rows=S)
-        log(f"case: prefill attention, {hpw} query heads per workgroup, S={S}")
-        outs[hpw] = to_np(vm.forward_hidden(x, None))
+        log(f"case: prefill attention, FDLLM_PREFILL_PAIR={pair} FDLLM_PREFILL_HPW={hpw}, S={S}")
+        outs[pair, hpw] = to_np(vm.forward_hidden(x, None))
         vm.close()
-    for hpw in (2, 3, 6):
-        np.testing.assert_array_equal(outs[hpw], outs[1])
+    for form in outs:
+        np.testing.assert_array_equal(outs[form], outs[0, 2], err_msg=str(form))
 
 
 def test_vm_from_artifact_equals_vm_from_tensors(tiny, tmp_path):
