@@ -202,7 +202,7 @@ static hipError_t launch_prefill_cfg(const AttnP& a, int paired, hipStream_t st)
 template <int DT, int MASK>
 static hipError_t launch_prefill(const AttnP& a, hipStream_t st) {
   if (!a.roped) hipLaunchKernelGGL(rope_kv_kernel<DT>, dim3(a.rows), dim3(128), 0, st, a);
-  const PrefillForm f = prefill_form(a.rows, a.nq, a.nkv, a.prefill_pair, a.prefill_hpw);
+  const PrefillForm f = prefill_form(a.rows, a.nq, a.nkv, a.cus, a.prefill_pair, a.prefill_hpw);
   return f.whole ? launch_prefill_cfg<DT, MASK, 3>(a, f.paired, st) : launch_prefill_cfg<DT, MASK, 1>(a, f.paired, st);
 }
 

@@ -345,6 +345,7 @@ int plan_attention(fdllm_ctx* c, AttnP& a, int rows, uint16_t* kc, uint16_t* vc,
     }
     target = std::max(1, target / sb->nseq);
   }
+  a.cus = c->ncu;
   a.ncu = c->seq_attn ? c->ncu : 0;
   const AttnPlan pl = attn_plan(a.rows, a.nq, a.nkv, a.Lk, target, a.nseq, mask, a.ncu);
   // batched calls without a mask take attn_seq_kernel (every key of a sequence in one workgroup, no

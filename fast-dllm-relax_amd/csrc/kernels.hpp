@@ -208,6 +208,7 @@ struct AttnP {
   // writes them there (it may be qkv itself: each row's heads are rotated in place)
   uint16_t* qrot; int ldqr;
   int xh;                             // attn_seq_kernel, one sequence: runs of query-tile groups (AttnPlan)
+  int cus;                            // compute units (prefill_form)
   int ncu;                            // compute units (attn_plan's splits of one sequence; 0: no attn_seq_kernel for it)
   // batched call (nseq > 1, chunked kernel only): sequence b owns rows [b rows, (b + 1) rows) of qkv,
   // rope and out, the cache at kc / vc + b seq_stride, writes from seq_ws[b] and attends

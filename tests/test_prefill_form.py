@@ -19,8 +19,8 @@ def form(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I", str(ROOT / "fast-dllm-relax_amd" / "csrc"),
                     str(ROOT / "tests" / "prefill_form_check.cpp"), "-o", str(exe)], check=True)
 
-    def get(*args):
-        out = subprocess.run([str(exe), *map(str, args)], capture_output=True, text=True, check=True)
+    def get(rows, nq, nkv, pair, hpw, cus=256):
+        out = subprocess.run([str(exe), *map(str, (rows, nq, nkv, cus, pair, hpw))], capture_output=True, text=True, check=True)
         whole, paired = out.stdout.split()
         return f"{'twelve' if whole == '1' else 'four'} {'paired' if paired == '1' else 'alone'}"
 
@@ -31,6 +31,7 @@ def test_forms_by_size(form):
     for rows, want in [(128, "four alone"), (1504, "four alone"), (1728, "four paired"), (2048, "four paired"),
                        (2880, "twelve alone"), (6000, "twelve alone"), (7168, "twelve paired"), (8192, "twelve paired")]:
         assert form(rows, 12, 2, 1, 0) == want, rows
+        assert form(rows // 2, 12, 2, 1, 0, cus=128) == want, (rows // 2, "of 128 compute units")
     assert form(8192, 4, 2, 1, 0) == "four paired"  # no group of six heads
 
 
