@@ -376,15 +376,10 @@ static hipError_t launch_wt_cfg(const GemmP& a, const GemmPlan& p, hipStream_t s
 template <int DT, int EPI, class W>
 static hipError_t launch_wk_cfg(const GemmP& a, const GemmPlan& p, hipStream_t st) {
   auto kern = gemm_wk_kernel<DT, EPI, W::mf, W::tpw, W::nwn, W::kp, W::d>;
-  if (a.KS % (p.ksplit * W::kp)) return hipErrorInvalidValue;
+  if (p.ksplit != 1 || a.KS % W::kp) return hipErrorInvalidValue;
   static_assert(W::lds <= 64 * 1024, "no LDS attribute needed");
   const int total = p.nbm * p.nbn, per = (total + 7) / 8;
-  hipLaunchKernelGGL(kern, dim3(8 * per, p.ksplit), dim3(64 * W::nwn * W::kp), W::lds, st, a, p.nbm, p.nbn);
-  if (p.ksplit > 1 && !a.part_rows) {
-    const int nblk = (a.M + 15) / 16;
-    hipLaunchKernelGGL((gemm_mm_split_epilogue_kernel<DT, EPI>), dim3((a.N + 15) / 16, (nblk + 3) / 4), dim3(256), 0,
-                       st, a, p.ksplit);
-  }
+  hipLaunchKernelGGL(kern, dim3(8 * per), dim3(64 * W::nwn * W::kp), W::lds, st, a, p.nbm, p.nbn);
   return hipGetLastError();
 }
 

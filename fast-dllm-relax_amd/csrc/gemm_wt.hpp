@@ -490,9 +490,8 @@ void gemm_wk_kernel(GemmP a, int nbm, int nbn) {
   constexpr int DPW = (MF + NWN - 1) / NWN;  // activation blocks each wave copies per stage (past the last: the last again)
   constexpr int VPS = TPW + DPW;             // vector memory instructions per wave per stage
   static_assert(D >= 2 && (D - 1) * VPS < 64, "outstanding copies fit the memory counter");
-  static_assert(EPI != EPI_SILU_PAIR || TPW % 2 == 0, "gate/up pairs stay within a wave");
+  static_assert(EPI == EPI_SILU_PAIR && TPW % 2 == 0, "gate_up; its pairs stay within a wave");
   static_assert(KP == 2 && MF % 2 == 0, "two groups, each finishing every other row block");
-  static_assert(EPI != EPI_LOGITS, "no confidence tiles here");
   extern __shared__ __align__(16) unsigned char smem[];  // [R][KP][MF][1 KB]
 
   const int total = nbm * nbn;
@@ -506,8 +505,7 @@ void gemm_wk_kernel(GemmP a, int nbm, int nbn) {
   const int lr = lane & 15, lg = lane >> 4;
   const int m0 = mb * 16 * MF, mlast = a.M - 1;
   const int tw0 = (nb * NWN + wn) * TPW, tlast = a.ntiles - 1;  // this wave's first tile
-  const int ks = a.KS / (int)gridDim.y, kb = (int)blockIdx.y * ks + kp;  // the split's k steps; this group's first
-  const int nst = ks / KP;  // (the plan takes whole stages)
+  const int nst = a.KS / KP;  // stages (the plan takes whole ones); the group's first k step is kp
 
   const u16* xs[DPW];
   size_t xstep[DPW];
@@ -516,17 +514,17 @@ void gemm_wk_kernel(GemmP a, int nbm, int nbn) {
     const int i = min(wn + NWN * q, MF - 1);
     if (a.xfrag == 2) {
       const int b = min(m0 / 16 + i, mlast / 16);
-      xs[q] = a.X + ((size_t)b * a.KS + kb) * 512 + 8 * lane;
+      xs[q] = a.X + ((size_t)b * a.KS + kp) * 512 + 8 * lane;
       xstep[q] = 512 * KP;
     } else {
       const int m = min(m0 + 16 * i + lr, mlast);
-      xs[q] = a.X + (size_t)m * a.ldx + 32 * kb + 8 * lg;
+      xs[q] = a.X + (size_t)m * a.ldx + 32 * kp + 8 * lg;
       xstep[q] = 32 * KP;
     }
   }
   const u16* ws[TPW];
 #pragma unroll
-  for (int j = 0; j < TPW; ++j) ws[j] = a.W + ((size_t)min(tw0 + j, tlast) * a.KS + kb) * 512 + 8 * lane;
+  for (int j = 0; j < TPW; ++j) ws[j] = a.W + ((size_t)min(tw0 + j, tlast) * a.KS + kp) * 512 + 8 * lane;
 
   u32x4 wv[R][TPW];
   auto issue = [&](int st, u32x4 (&dst)[TPW], int buf) {
@@ -603,21 +601,10 @@ void gemm_wk_kernel(GemmP a, int nbm, int nbn) {
         }
         acc[j][f] = sum;
       }
-      if (gridDim.y > 1) {
 #pragma unroll
-        for (int j = 0; j < TPW; ++j) store_split_unit(a, blockIdx.y, tw0 + j, mb * MF + f, lane, acc[j][f]);
-      } else if constexpr (EPI == EPI_SILU_PAIR) {
-#pragma unroll
-        for (int p = 0; p < TPW / 2; ++p) {
-          const f32x4 v[2] = {acc[2 * p][f], acc[2 * p + 1][f]};
-          os_epilogue<DT, EPI, 2, false>(a, v, m0 + 16 * f + lr, tw0 + 2 * p, lg);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < TPW; ++j) {
-          const f32x4 v[1] = {acc[j][f]};
-          os_epilogue<DT, EPI, 1, false>(a, v, m0 + 16 * f + lr, tw0 + j, lg);
-        }
+      for (int p = 0; p < TPW / 2; ++p) {
+        const f32x4 v[2] = {acc[2 * p][f], acc[2 * p + 1][f]};
+        os_epilogue<DT, EPI, 2, false>(a, v, m0 + 16 * f + lr, tw0 + 2 * p, lg);
       }
     }
   });

@@ -148,7 +148,7 @@ inline int mm_choice(int cfg, int M, int ntiles, int ks, const MmPolicy& pol) {
     // 20.5, 64 rows 18.5 / 21.0 / 22.7, 96 rows 20.5 / - / 24.1, 128 rows 23.3 / 29.9 / 26.0, 129 rows 30.8 / 27.2 /
     // 31.6, 192 rows 32.5 / 28.8 / 34.2, 208 rows - / 34.5 / 35.0, 256 rows 37.6 / 37.5 / 37.1 / 43.2, 320 rows - / 37.8
     // / 34.9 / 41.7, 384 rows - / 43.2 / 36.6 / 42.1, 416 rows - / 44.3 / 43.0 / 42.0, 512 rows - / 54.1 / 48.8 / 42.6
-    if (M <= 128 && ntiles % 6 == 0) return M <= 64 ? MM_WK_GU4 : M <= 96 ? MM_WK_GU6 : MM_WK_GU8;
+    if (M <= 128) return M <= 64 ? MM_WK_GU4 : M <= 96 ? MM_WK_GU6 : MM_WK_GU8;
     if (M <= 224) return MM_WR_S;
     // (2048 x 11008, 519 blocks of 128 x 128 for two workgroups per unit: 53.7 / 51.7 LDS-staged at 300 rows)
     if (M <= 400 && mm_blocks(MM_WR_M, M, ntiles) <= 2 * pol.cus) return MM_WR_M;
