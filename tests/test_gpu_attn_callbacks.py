@@ -1,8 +1,8 @@
 """fdllm_attn_inplace and fdllm_kv_write, the reference's attention callbacks fast_dllm.attn_inplace and
 fast_dllm.kv_write (fast_dllm_relax/runtime.py:19-80), against the oracle's restatement
-(OracleModel.attn_inplace / kv_write), through the C ABI.  Every case names the kernel family its row
-count takes: the chunk kernel (up to 32 rows), the loop kernel (33 to 127) and the prefill kernel (128
-rows and more, queries staged in the output buffer)."""
+(OracleModel.attn_inplace / kv_write), through the C ABI.  Every case names the kernel its row and
+key counts take: the chunk kernel (up to 32 rows over up to 5120 keys), attn_seq_kernel (up to 1023 rows) and the
+prefill kernel (1024 rows and more, queries staged in the output buffer)."""
 
 from __future__ import annotations
 
@@ -73,8 +73,10 @@ def _case(ref, vm, rows, P, write_rel, attend_rel, cap, seed, layer):
     (32, 96, 0, 32, 160),      # the full block step's call: chunk kernel
     (8, 96, 8, 32, 160),       # a partial step (rp 8): chunk kernel
     (32, 2016, 0, 32, 2080),   # the config-3 prefix: chunk kernel, 16 key chunks + merge
-    (64, 40, 0, 64, 128),      # a scoring tail: loop kernel
-    (160, 32, 0, 160, 192),    # prefill kernel with the queries staged in out
+    (64, 40, 0, 64, 128),      # a scoring tail: attn_seq_kernel
+    (160, 32, 0, 160, 192),    # a longer one
+    (8, 5200, 8, 32, 5248),    # a partial step past the chunk kernel's keys: attn_seq_kernel in key splits
+    (1050, 31, 0, 1050, 1088), # prefill kernel with the queries staged in out
     (32, 64, 0, 80, 128),      # attended rows past the capacity: the reference's slice stops at cap
     (20, 50, 3, 30, 96),       # unaligned window and row count
 ])

@@ -232,7 +232,7 @@ def test_seq_attention_kernel_matches_chunk_kernel(monkeypatch):
 def test_batched_step_beyond_one_step_key_split_plan(wide2):
     """A batched call whose longest prefix (8300 keys) is past the chunk kernel's one-step plan (64 chunks of
     128 keys): attn_seq_kernel streams every key, so the call runs; each sequence's hidden states match the
-    batch-1 cached forward of the same sequence (the long-block loop kernel) to the bf16 criterion."""
+    batch-1 cached forward of the same sequence (its own key splits of that kernel) to the bf16 criterion."""
     _, vm = wide2
     kw = WIDE2
     rng = np.random.default_rng(43)

@@ -7,10 +7,10 @@ test_gpu_loop.py; config 2 at full depth in test_gpu_fulldepth.py.)
   batched path's default attention (the RoPE / KV-append pass and attn_seq_kernel with key splits over the
   idle compute units, merged by the last split to arrive), the 8-row partial step the chunk kernel; each
   sequence's hidden states and appended K/V rows meet the per-sequence fp16 oracle.
-* Config 5: bf16, seed 4, an 8192-token prefix through build_prefix_cache (the paired-query-block prefill
-  attention in its default regime and the register-weight GEMMs at M = 8192) against the oracle's caches,
+* Config 5: bf16, seed 4, an 8192-token prefix through build_prefix_cache (the prefill attention on paired
+  query blocks, its default there, and the register-weight GEMMs at M = 8192) against the oracle's caches,
   then the 64-token continuation scored by score_masked_continuation (64 cached rows: 24 query tiles per
-  kv head, the long-block attention kernel with key splits) and its per-token log-probabilities.
+  kv head, attn_seq_kernel in key splits) and its per-token log-probabilities.
 """
 
 from __future__ import annotations

@@ -1,12 +1,12 @@
 """The register-weight large-M GEMM against the LDS-staged and streaming large-M GEMMs.
 
-By default gate_up and down run gemm_wr_kernel's 128 x 256 blocks from 2048 rows and qkv and o_proj from
-4096 (FDLLM_WR_OPS selects the projections, one bit per GemmCfg; FDLLM_WR_MIN_ROWS lowers the threshold,
-here to 256 so that ragged and small row counts take it too); below that qkv, and o_proj below 2048 rows,
-run its 64 x 128 blocks, or up to 512 rows its 64 x 64 blocks (FDLLM_WR_SMALL, bits of qkv and o_proj).  Every large-M kernel accumulates each
-output element's k steps in order in one MFMA chain and shares the epilogues, so with k splits off
-(FDLLM_MM_TARGET_WGS=1) the hidden states must agree bit for bit whichever kernel ran.  Parity of the default configuration with the oracle is
-established by the prefill, forward_hidden and batched-step tests."""
+By default the projections run gemm_wr_kernel's large blocks (128 x 256, 128 x 192) where mm_choice.hpp's counts say so
+(FDLLM_WR_OPS selects the projections, one bit per GemmCfg; FDLLM_WR_MIN_ROWS replaces the counts by a row threshold,
+here 256 so that ragged and small row counts take it too); below that qkv, and o_proj while they make one round,
+run its 64 x 128 blocks, or up to 512 rows its 64 x 64 blocks (FDLLM_WR_SMALL, bits of qkv and o_proj).  Every large-M
+kernel accumulates each output element's k steps in order in one MFMA chain and shares the epilogues, so with k splits
+off (FDLLM_MM_TARGET_WGS=1) the hidden states must agree bit for bit whichever kernel ran.  Parity of the default
+configuration with the oracle is established by the prefill, forward_hidden and batched-step tests."""
 
 from __future__ import annotations
 
@@ -112,20 +112,21 @@ def _prefill_vm(kw, params, dtype, monkeypatch, pair, max_rows):
     from fast_dllm_relax_amd.vm import HipVM
 
     monkeypatch.setenv("FDLLM_PREFILL_PAIR", str(pair))
+    monkeypatch.setenv("FDLLM_SEQ_ATTN", "0")  # (the unmasked call of 200 rows would take attn_seq_kernel)
     vm = HipVM(FastDLLMConfig(**kw), params, dtype=dtype, max_rows=max_rows)
     monkeypatch.delenv("FDLLM_PREFILL_PAIR")
+    monkeypatch.delenv("FDLLM_SEQ_ATTN")
     return vm
 
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 def test_prefill_pair_kernel_bit_identical(dtype, monkeypatch):
-    """The paired-query-block prefill attention, with all six heads of a kv head per workgroup
-    (FDLLM_PREFILL_PAIR=2 forces it at every size; by default it runs once its workgroups fill the chip,
-    from 4096 rows) and with the heads split over three workgroups (=3 forces it; by default from 32
-    query blocks below that), against attn_prefill_kernel: the same key blocks in the same order per query,
-    so hidden states and caches agree bit for bit.  Odd and even query-block counts, a ragged last block,
-    the block-causal mask (forward_hidden, build_prefix_cache) and the unmasked form (a cached forward of
-    200 rows after a prefix)."""
+    """attn_prefill_kernel on paired query blocks, with all six heads of a kv head per workgroup
+    (FDLLM_PREFILL_PAIR=2 forces it at every size; by default it runs once its workgroups fill the chip) and with
+    the heads split over three workgroups (=3 forces it), against single blocks (=0): the same key blocks in the
+    same order per query, so hidden states and caches agree bit for bit.  Odd and even query-block counts, a ragged
+    last block, the block-causal mask (forward_hidden, build_prefix_cache) and the unmasked form (a cached forward
+    of 200 rows after a prefix)."""
     from fast_dllm_relax_amd.config import FastDLLMConfig
     from fast_dllm_relax_amd.params import from_numpy
     from oracle.model import OracleConfig, random_params
@@ -211,7 +212,7 @@ def test_lm_head_register_weight_bit_identical(dtype, monkeypatch):
 def test_fused_down_norm_bit_identical(dtype, monkeypatch):
     """A large-M down launch that splits k hands its split sums, row-major, to resid_norm_kernel, which adds
     them, applies the residual epilogue and the next RMSNorm (the next layer's qkv input, or the final norm)
-    in one launch; up to 256 rows o_proj does the same with three k splits (the post-attention norm).  The
+    in one launch; up to 256 rows o_proj does the same with forced k splits (the post-attention norm).  The
     arithmetic is the split-sum kernel's and norm_rows_kernel's, and k splits add their sums in split order,
     so the results match the separate launches (FDLLM_FUSE_DOWN=0, FDLLM_FUSE_OPROJ=0) except where o_proj's
     forced split regroups its fp32 sums: the hidden states at sizes that fuse only down, and the caches and

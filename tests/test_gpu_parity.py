@@ -385,7 +385,7 @@ def test_vm_from_artifact_equals_vm_from_tensors(tiny, tmp_path):
 
 def test_long_context_prefill_and_cached_step(tiny):
     """A prefix past 64 key chunks of 128 (P = 8200, ragged): the prefill kernel over 8200 rows, then a
-    32-row cached step whose attention takes the split loop kernel (more than 64 chunks), vs the oracle."""
+    32-row cached step whose attention takes attn_seq_kernel in key splits, vs the oracle."""
     ref, vm = tiny
     from oracle.model import OracleModel
 

@@ -83,9 +83,9 @@ def test_prefill_attention_block_causal(dtype):
         blk = (rows - 1) // 32 * 32
         bias = torch.from_numpy(build_prefix_block_attention_bias(blk, rows - blk, block_size=32)).cuda()
         log(f"case: block-causal {rows} rows, {dtype}")
-        a, b = vm.forward_hidden(x, None).double(), vm.forward_hidden(x, bias).double()
-        # two layers of rounded tensors: each rounding (about 10 per layer) may flip by an ulp
-        assert float((a - b).norm() / b.norm()) < 4 * ULP2[dtype], rows
+        a, b = vm.forward_hidden(x, None)[0].double(), vm.forward_hidden(x, bias)[0].double()
+        # two layers of rounded tensors: each rounding (about 10 per layer) may flip by an ulp, in any row
+        assert float(((a - b).norm(dim=1) / b.norm(dim=1)).max()) < 4 * ULP2[dtype], rows
 
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
