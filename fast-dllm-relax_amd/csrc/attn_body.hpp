@@ -1155,7 +1155,7 @@ void attn_prefill_kernel(AttnP a, int paired) {
 // x of NQW query tiles) with NQW KH waves: wave w takes query tile NQW x + w % NQW of the stacked rows of
 // the chunk kernels (row qi = head in group x rows + r, 16 per tile) and key part kh = w / NQW, i.e. keys
 // 64 j + 64 / KH kh .. of every block j of the split (keys past Lk_b masked).  The blocks stream through
-// LDS, D blocks ahead, by the global-to-LDS copy in the paired prefill kernel's layout (a 256-byte row per
+// LDS, D blocks ahead, by the global-to-LDS copy in the prefill kernel's layout (a 256-byte row per
 // key, 16-byte chunk c of row r at slot c ^ (r % 16); V^T fragments from the transposing LDS read).
 // rope_kv_kernel has already appended this call's K/V rows to the cache and put the RoPE'd queries in
 // out, so every key comes from the cache and each query is read from out before its output is written
@@ -1168,7 +1168,7 @@ void attn_prefill_kernel(AttnP a, int paired) {
 // One sequence's unmasked call (nseq <= 1: scoring, a block after more keys than the chunk kernel takes)
 // runs here too, split into p.S equal ranges of key blocks whose partials attn_merge_kernel combines: the
 // loop kernel it replaces aimed for 64 workgroups and waited out a memory round trip per 32 keys (83 rows
-// over 8275 keys: 168 -> 23 us; 32 rows: 47 -> 23).  What bounds it is the serial chain of a block in one
+// over 8275 keys: 168 -> 23 us; 32 rows over 8207: 47 -> 16.4).  What bounds it is the serial chain of a block in one
 // wave per SIMD (scores, softmax, P.V: about 1 us per 64 keys), not the 8.5 MB of K and V.
 // 1-D grid in XCD-aware order: linear index i, slot i % 8, round i / 8; pair (u, g) = (round / XG) x 8 +
 // slot, query group x = round % XG, so the XG workgroups that read one split's K/V run on one XCD and

@@ -107,10 +107,12 @@ struct fdllm_ctx {
   unsigned* attn_cnt = nullptr;  // attn_seq_kernel's arrival counters (SEQ_CNT_MAX, zero between launches)
   int fuse_down = 1;      // large-M down launches with k splits: split sum + residual + next RMSNorm in one launch
   // large-M o_proj with a forced k split and its split sum + residual + the next norm in one launch: -1 with
-  // three or two splits up to 256 and from 513 rows, where that many of its blocks make one round of the compute
-  // units (us per layer of a prefill, two / three splits / none: 192 rows 67.6 / 67.0 / -, 200 rows 66.6 / 68.6 / -,
-  // 400 rows 88.7 / 87.9 / 87.1, 576 rows 96.4 / 98.7 / 100.1, 672 rows 115.3 / 114.5 / 114.0), 0 never, N > 1 with N
-  // splits at any size
+  // three or two splits where that many of its blocks make one round of the compute units, but not from 257 to 512
+  // rows: from 350 on its blocks are faster unsplit there, and below, where two splits would save 2 percent, the call
+  // keeps the unsplit sums' bits (a 300-row call is tested for them).  us per layer of a prefill, two / three splits /
+  // none: 192 rows 82.8 / 81.9 / 87.2, 256 rows 88.8 / 92.1 / 93.3, 300 rows 93.2 / 96.2 / 95.1, 350 rows 101.1 / 99.7 /
+  // 98.8, 400 rows 110.4 / 109.0 / 107.7, 512 rows 113.5 / 115.6 / 110.8, 576 rows 119.4 / 121.9 / 124.1, 640 rows 124.3 /
+  // 127.6 / 128.6, 672 rows 134.6 / 134.0 / 133.6.  0 never, N > 1 with N splits at any size
   int fuse_oproj = -1;
   // large-M calls whose attention starts with the RoPE / KV-append pass (prefill, batched sequences): that
   // pass done by qkv's epilogue instead (FDLLM_QKV_ROPE=0: the separate pass)
@@ -1043,8 +1045,8 @@ int fdllm_kv_write(fdllm_ctx* c, const void* k, const void* v, int rows, void* k
 // (already rotated) queries over cache rows [0, prefix_len + attend_rel) with no mask (_attend,
 // runtime.py:30-48).  The chunk kernel and attn_seq_kernel take the queries from q (AttnP::rope null: no
 // RoPE); the chunk kernel also takes and writes the K/V rows, the others find them in the cache (ws = Lk: no
-// rows of the call are read from q's buffer or appended); the prefill kernels (1024 rows and more) read rotated queries from the output buffer, where they
-// are copied first.
+// rows of the call are read from q's buffer or appended); the prefill kernel (1024 rows and more) reads rotated
+// queries from the output buffer, where they are copied first.
 int fdllm_attn_inplace(fdllm_ctx* c, const void* q, const void* k, const void* v, int rows, void* k_cache,
                        void* v_cache, int cap, int layer, int64_t prefix_len, int write_rel, int attend_rel, void* out,
                        void* stream) {

@@ -482,7 +482,7 @@ void gemm_wr_kernel(GemmP a, int nbm, int nbn) {
 // For calls of 33 to 128 rows, whose launches are bound by what a compute unit takes in: (rows + columns) x 3 KB
 // per workgroup at hidden 1536.  Columns are chosen so that one round of workgroups covers the chip with as few
 // bytes each as possible, and the k groups put more waves, hence more loads in flight, on each compute unit
-// than the columns alone would (figures at mm_choice).
+// than the columns alone would (figures at mm_choice, mm_choice.hpp).
 template <int DT, int EPI, int MF, int TPW, int NWN, int KP, int D>
 __global__ __launch_bounds__(64 * NWN * KP) __attribute__((amdgpu_waves_per_eu((NWN * KP + 3) / 4, (NWN * KP + 3) / 4)))
 void gemm_wk_kernel(GemmP a, int nbm, int nbn) {

@@ -70,7 +70,8 @@ constexpr MmInfo mm_info(int id) {
 #ifndef FD_WR_LM_MIN_ROWS
 #define FD_WR_LM_MIN_ROWS 256
 #endif
-// Rows from which a projection takes the register-weight kernel by default.  Measured (1.5B, us per
+// Rows from which a projection takes the register-weight kernel by default, where the counts in mm_choice have not
+// decided before.  Measured (1.5B, us per
 // launch, register-weight / previous kernel): gate_up 53 / 47 at 512 rows, 110 / 118 at 2048, 377 / 448
 // at 8192; down 40 / 30, 79 / 80, 189 / 192; qkv 37 / 31 at 2048, 75 / 106 at 8192; o_proj 38 / 23,
 // 57 / 70.  Below these sizes its 128 x 256 blocks leave too few workgroups without a k split.
